@@ -485,12 +485,21 @@ static int ensure_n2e(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m) {
       const int64_t v = mesh->h_conn[size_t(e * nen + a)] - 1;
       lst[size_t(fill[size_t(v)]++)] = int32_t((e << 5) | a);
     }
-  GF_HIP_CHECK(ctx, hipMalloc(&m->d_n2e_ptr, ptr.size() * sizeof(int64_t)));
-  GF_HIP_CHECK(ctx, hipMalloc(&m->d_n2e, std::max<size_t>(lst.size(), 1) * sizeof(int32_t)));
-  GF_HIP_CHECK(ctx, hipMemcpy(m->d_n2e_ptr, ptr.data(), ptr.size() * sizeof(int64_t),
-                              hipMemcpyHostToDevice));
-  GF_HIP_CHECK(ctx, hipMemcpy(m->d_n2e, lst.data(), lst.size() * sizeof(int32_t),
-                              hipMemcpyHostToDevice));
+  int64_t* d_ptr = nullptr;
+  int32_t* d_lst = nullptr;
+  hipError_t e = hipMalloc(&d_ptr, ptr.size() * sizeof(int64_t));
+  if (e == hipSuccess) e = hipMalloc(&d_lst, std::max<size_t>(lst.size(), 1) * sizeof(int32_t));
+  if (e == hipSuccess)
+    e = hipMemcpy(d_ptr, ptr.data(), ptr.size() * sizeof(int64_t), hipMemcpyHostToDevice);
+  if (e == hipSuccess)
+    e = hipMemcpy(d_lst, lst.data(), lst.size() * sizeof(int32_t), hipMemcpyHostToDevice);
+  if (e != hipSuccess) {  // nothing half-built is left behind
+    if (d_ptr) (void)hipFree(d_ptr);
+    if (d_lst) (void)hipFree(d_lst);
+    return set_error(ctx, GF_ERR_HIP, std::string("node incidence: ") + hipGetErrorString(e));
+  }
+  m->d_n2e_ptr = d_ptr;
+  m->d_n2e = d_lst;
   return GF_OK;
 }
 
@@ -597,6 +606,30 @@ static int assemble_with(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m, int varian
   return GF_OK;
 }
 
+// the element tensors (variant 2) must leave most of the device free
+static bool tensors_fit(const gf_mesh* mesh) {
+  size_t free_b = 0, total_b = 0;
+  const double need = double(elem_tensor_doubles(mesh->type, mesh->nelem)) * sizeof(double);
+  return hipMemGetInfo(&free_b, &total_b) == hipSuccess && need <= 0.5 * double(free_b);
+}
+
+// The assembly kernel of a mesh too small to be worth timing (below 65536
+// elements), 3D: the node gather, for the 20-node brick over the element
+// tensors of the matrix cores, as the tuner picks them on every large mesh.
+// One or two launches that write each value once, where the colored scatter
+// takes a launch per color, clears the ELL values first and re-lays them out
+// for the solver afterwards.  Measured, a pass with the copy kept current:
+// Brick20 30x33x28 1.06 ms against 3.92 ms (24x24x24 0.55 / 1.99, 20x17x13
+// 0.20 / 0.73); Brick8 64x32x32 0.149 / 0.625.  The scatter stays for nodes
+// with more neighbours than the gather holds, and in 2D: it sums the Gauss
+// points in the reference's order, and on slender plates (Q8 128x8, condition
+// number 1.5e8) the other rounding of the gather's entries moves the solution
+// by 1e-9, for 0.02 ms of a pass saved (Q4 64x32: 0.010 / 0.032 ms).
+static int small_mesh_variant(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m) {
+  if (mesh->dim != 3 || !gather_fits(mesh, m) || ensure_n2e(ctx, mesh, m) != GF_OK) return 0;
+  return mesh->type == GF_BRICK20 && tensors_fit(mesh) ? 2 : 3;
+}
+
 static int check_assembly_args(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m, const char* fn) {
   if (!ctx || !mesh || !m) return set_error(ctx, GF_ERR_ARG, std::string(fn) + ": null argument");
   if (m->ncolors == 0 || m->nelem != mesh->nelem || m->nen != mesh->nen ||
@@ -644,12 +677,7 @@ int gf_assemble_tune(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m, int32_t force,
     for (int v : {0, 1, 3, 2}) {
       if ((v == 3 || v == 2) && !gather_fits(mesh, m)) continue;
       if (v == 2 && mesh->type != GF_BRICK20) continue;
-      if (v == 2 && !m->d_etens) {
-        // the tensors must leave most of the device free: else not tried
-        size_t free_b = 0, total_b = 0;
-        const double need = double(elem_tensor_doubles(mesh->type, mesh->nelem)) * sizeof(double);
-        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || need > 0.5 * double(free_b)) continue;
-      }
+      if (v == 2 && !m->d_etens && !tensors_fit(mesh)) continue;
       gf_timing t1{}, t2{};
       if ((st = assemble_with(ctx, mesh, m, v, &t1)) || (st = assemble_with(ctx, mesh, m, v, &t2)))
         return st;
@@ -675,8 +703,8 @@ int gf_assemble(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m, gf_timing* t) {
   int st = check_assembly_args(ctx, mesh, m, "gf_assemble");
   if (st) return st;
   if (m->asm_variant < 0) {
-    // small meshes: not worth timing; large ones pick the faster kernel once
-    if (m->nelem < 65536) m->asm_variant = 0;
+    // small meshes: not worth timing; large ones pick the fastest kernel once
+    if (m->nelem < 65536) m->asm_variant = small_mesh_variant(ctx, mesh, m);
     else if ((st = gf_assemble_tune(ctx, mesh, m, -1, nullptr, nullptr))) return st;
   }
   return assemble_with(ctx, mesh, m, m->asm_variant, t);

@@ -197,7 +197,8 @@ int gf_assemble(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m, gf_timing* t);
  * fit); -1 assembles twice with each of 0, 1, 3 and, for Brick20 when its
  * tensors take at most half the free device memory, 2, and keeps the
  * fastest (gf_assemble does this on its first call for meshes of 65536
- * elements or more).  When the solver's block-sliced copy of the matrix
+ * elements or more; smaller ones take 3 for Brick8, 2 for Brick20, else 0,
+ * untimed).  When the solver's block-sliced copy of the matrix
  * exists, 2, 3 and 4 write it with only the diagonal of the ELL values
  * (the other ELL values are rebuilt from the copy by the first call that
  * reads them) and the others are followed by the copy, inside the
