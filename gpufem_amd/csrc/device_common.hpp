@@ -26,6 +26,27 @@ __device__ inline double block_sum(double v, double* sh) {
   return t;
 }
 
+// Two of them at once (sh: 2 * kNT / 64).
+__device__ inline void block_sum2(double* a, double* b, double* sh) {
+  double va = *a, vb = *b;
+  for (int off = 32; off > 0; off >>= 1) {
+    va += __shfl_xor(va, off);
+    vb += __shfl_xor(vb, off);
+  }
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) {
+    sh[threadIdx.x >> 6] = va;
+    sh[kNT / 64 + (threadIdx.x >> 6)] = vb;
+  }
+  __syncthreads();
+  *a = *b = 0.0;
+#pragma unroll
+  for (int w = 0; w < kNT / 64; ++w) {
+    *a += sh[w];
+    *b += sh[kNT / 64 + w];
+  }
+}
+
 // Sum of np per-block partials, identical in every workgroup (a fixed order:
 // four strided accumulators per thread, so four loads are in flight when the
 // SpMV grid leaves thousands of partials).
@@ -41,6 +62,46 @@ __device__ inline double reduce_partials(const double* part, int np, double* sh)
   if (i + kNT < np) v[1] += part[i + kNT];
   if (i + 2 * kNT < np) v[2] += part[i + 2 * kNT];
   return block_sum((v[0] + v[1]) + (v[2] + v[3]), sh);
+}
+
+// Two such sums over np partials each, their loads in flight together (one
+// memory latency and one workgroup barrier; sh: 2 * kNT / 64, not in use by a
+// wave that still reads it).  The first kNT threads of the workgroup add, so
+// workgroups of any size get reduce_partials' own sums, bitwise.
+__device__ inline void reduce_partials2(const double* pa, const double* pb, int np, double* sa,
+                                        double* sb, double* sh) {
+  double a[4] = {0.0, 0.0, 0.0, 0.0}, b[4] = {0.0, 0.0, 0.0, 0.0};
+  int i = threadIdx.x < kNT ? threadIdx.x : np;
+  for (; i + 3 * kNT < np; i += 4 * kNT) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      a[u] += pa[i + u * kNT];
+      b[u] += pb[i + u * kNT];
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < 3; ++u) {
+    if (i + u * kNT < np) {
+      a[u] += pa[i + u * kNT];
+      b[u] += pb[i + u * kNT];
+    }
+  }
+  double va = (a[0] + a[1]) + (a[2] + a[3]), vb = (b[0] + b[1]) + (b[2] + b[3]);
+  for (int off = 32; off > 0; off >>= 1) {
+    va += __shfl_xor(va, off);
+    vb += __shfl_xor(vb, off);
+  }
+  if ((threadIdx.x & 63) == 0 && threadIdx.x < kNT) {
+    sh[threadIdx.x >> 6] = va;
+    sh[kNT / 64 + (threadIdx.x >> 6)] = vb;
+  }
+  __syncthreads();
+  *sa = *sb = 0.0;
+#pragma unroll
+  for (int w = 0; w < kNT / 64; ++w) {
+    *sa += sh[w];
+    *sb += sh[kNT / 64 + w];
+  }
 }
 
 // Workgroups are dispatched round-robin over the 8 XCDs; the remap gives
@@ -136,9 +197,16 @@ __device__ inline T row_dot_node(int64_t i, int64_t n, const T* __restrict__ val
   return acc;
 }
 
+// a load that leaves the line in the caches (NT = false) or streams past them
+template <bool NT, class P>
+__device__ inline P load_as(const P* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+
 // the d*d values of block slot b for this lane, 16 bytes per load: FP64
 // pairs (bsell_vidx) or FP32 quads (bsell_vidx32)
-template <int D, class T>
+template <int D, class T, bool NT = true>
 __device__ inline void load_block(const T* __restrict__ bval, int64_t b, int lane, T* v) {
   constexpr int DD = D * D;
   const T* base = bval + b * DD * 64;
@@ -146,23 +214,23 @@ __device__ inline void load_block(const T* __restrict__ bval, int64_t b, int lan
     typedef double P2 __attribute__((ext_vector_type(2)));
 #pragma unroll
     for (int kp = 0; kp < DD / 2; ++kp) {
-      const P2 pr = __builtin_nontemporal_load(reinterpret_cast<const P2*>(base) + kp * 64 + lane);
+      const P2 pr = load_as<NT>(reinterpret_cast<const P2*>(base) + kp * 64 + lane);
       v[2 * kp] = pr.x;
       v[2 * kp + 1] = pr.y;
     }
-    if constexpr (DD & 1) v[DD - 1] = __builtin_nontemporal_load(base + (DD - 1) * 64 + lane);
+    if constexpr (DD & 1) v[DD - 1] = load_as<NT>(base + (DD - 1) * 64 + lane);
   } else {
     typedef float P4 __attribute__((ext_vector_type(4)));
 #pragma unroll
     for (int kq = 0; kq < DD / 4; ++kq) {
-      const P4 q = __builtin_nontemporal_load(reinterpret_cast<const P4*>(base) + kq * 64 + lane);
+      const P4 q = load_as<NT>(reinterpret_cast<const P4*>(base) + kq * 64 + lane);
       v[4 * kq] = q.x;
       v[4 * kq + 1] = q.y;
       v[4 * kq + 2] = q.z;
       v[4 * kq + 3] = q.w;
     }
 #pragma unroll
-    for (int k = DD & ~3; k < DD; ++k) v[k] = __builtin_nontemporal_load(base + k * 64 + lane);
+    for (int k = DD & ~3; k < DD; ++k) v[k] = load_as<NT>(base + k * 64 + lane);
   }
 }
 
@@ -177,9 +245,11 @@ struct VecOf<float, 2> {
   using type = float2;
 };
 
-// the d entries x[c .. c + d - 1] of one node (one vector load when d = 2)
+// the d entries of one node of a vector x[d * node + e] (one vector load when
+// d = 2)
 template <int D, class T>
-__device__ inline void load_node(const T* __restrict__ x, int64_t c, T* xv) {
+__device__ inline void load_node(const T* x, int32_t node, T* xv) {
+  const int64_t c = int64_t(node) * D;
   if constexpr (D == 2) {
     const auto v = *reinterpret_cast<const typename VecOf<T, 2>::type*>(x + c);
     xv[0] = v.x;
@@ -188,6 +258,34 @@ __device__ inline void load_node(const T* __restrict__ x, int64_t c, T* xv) {
 #pragma unroll
     for (int e = 0; e < D; ++e) xv[e] = x[c + e];
   }
+}
+
+// A direction that is not stored: p = z + beta p_old, formed wherever it is
+// read.  z and p_old are component-major (entry e of a node at e * nodes +
+// node), so the lanes of a wave, whose columns are consecutive nodes on most
+// meshes, read whole 64-byte pieces: node-major pairs (z, p_old) of 16 bytes
+// cost 1.36x the product (Brick8 96^3, 411 against 302 us), component-major
+// ones 1.07x.
+template <int D>
+struct LazyDirection {
+  const double* __restrict__ z;
+  const double* __restrict__ p;
+  int64_t nodes;
+  double beta;
+  // 32-bit byte offsets from a uniform base (the matrix fits the last-level
+  // cache: far fewer than 2^29 nodes) keep the addresses out of the registers
+  __device__ inline double at(int32_t node, int e) const {
+    const uint32_t off = uint32_t(node) * 8u;
+    const char* zb = reinterpret_cast<const char*>(z + e * nodes);
+    const char* pb = reinterpret_cast<const char*>(p + e * nodes);
+    return *reinterpret_cast<const double*>(zb + off) +
+           beta * *reinterpret_cast<const double*>(pb + off);
+  }
+};
+template <int D>
+__device__ inline void load_node(const LazyDirection<D>& x, int32_t node, double* xv) {
+#pragma unroll
+  for (int e = 0; e < D; ++e) xv[e] = x.at(node, e);
 }
 
 // Node row R of the block-sliced copy, lane l of slice s: acc[r] = (K x)_{dR+r}
@@ -210,30 +308,28 @@ __device__ inline void load_node(const T* __restrict__ x, int64_t c, T* xv) {
 // definite: a plain FP32 copy of a structured mesh repeats the same rounding
 // in every row, which shifts every eigenvalue by about the same amount.
 // Padding slots point at the row's own node and hold zeros (adding 0).
-template <int D, class T, bool OFF>
-__device__ inline int64_t bsell_col(const int32_t* __restrict__ bcol,
+template <bool OFF, bool NT>
+__device__ inline int32_t bsell_col(const int32_t* __restrict__ bcol,
                                     const int16_t* __restrict__ coff, int32_t base, int64_t b,
                                     int lane) {
-  if constexpr (OFF)
-    return int64_t(base + int32_t(__builtin_nontemporal_load(coff + b * 64 + lane))) * D;
-  else
-    return int64_t(__builtin_nontemporal_load(bcol + b * 64 + lane)) * D;
+  if constexpr (OFF) return base + int32_t(load_as<NT>(coff + b * 64 + lane));
+  else return load_as<NT>(bcol + b * 64 + lane);
 }
 
-template <int D, class T, bool OFF, bool DIFF = false>
+// X: a vector (pointer) or a LazyDirection
+template <int D, class T, bool OFF, bool DIFF = false, int U = (D == 2 ? 4 : 3), bool NT = true,
+          class X>
 __device__ inline void bsell_row(const BsellView& bs, const T* __restrict__ bval,
                                  const int32_t* __restrict__ bcol, int64_t b0, int32_t cnt,
-                                 int lane, const T* __restrict__ x, T* acc, int32_t base,
-                                 int32_t row = 0) {
-  constexpr int U = D == 2 ? 4 : 3;
+                                 int lane, const X x, T* acc, int32_t base, int32_t row = 0) {
 #pragma unroll
   for (int r = 0; r < D; ++r) acc[r] = T(0);
   T xr[D];
-  if constexpr (DIFF) load_node<D, T>(x, int64_t(row) * D, xr);
+  if constexpr (DIFF) load_node<D>(x, row, xr);
   // x_J - x_R off the diagonal, x_R on it
-  auto rel = [&](int64_t c, T* xv) {
+  auto rel = [&](int32_t c, T* xv) {
     if constexpr (DIFF) {
-      if (c != int64_t(row) * D) {
+      if (c != row) {
 #pragma unroll
         for (int e = 0; e < D; ++e) xv[e] -= xr[e];
       }
@@ -242,13 +338,13 @@ __device__ inline void bsell_row(const BsellView& bs, const T* __restrict__ bval
   int32_t j = 0;
   for (; j + U <= cnt; j += U) {
     T xv[U][D], v[U][D * D];
-    int64_t cu[U];
+    int32_t cu[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int64_t b = b0 + j + u;
-      cu[u] = bsell_col<D, T, OFF>(bcol, bs.coff, base, b, lane);
-      load_block<D, T>(bval, b, lane, v[u]);
-      load_node<D, T>(x, cu[u], xv[u]);
+      cu[u] = bsell_col<OFF, NT>(bcol, bs.coff, base, b, lane);
+      load_block<D, T, NT>(bval, b, lane, v[u]);
+      load_node<D>(x, cu[u], xv[u]);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -261,15 +357,82 @@ __device__ inline void bsell_row(const BsellView& bs, const T* __restrict__ bval
   }
   for (; j < cnt; ++j) {
     const int64_t b = b0 + j;
-    const int64_t c = bsell_col<D, T, OFF>(bcol, bs.coff, base, b, lane);
+    const int32_t c = bsell_col<OFF, NT>(bcol, bs.coff, base, b, lane);
     T xv[D], v[D * D];
-    load_block<D, T>(bval, b, lane, v);
-    load_node<D, T>(x, c, xv);
+    load_block<D, T, NT>(bval, b, lane, v);
+    load_node<D>(x, c, xv);
     rel(c, xv);
 #pragma unroll
     for (int r = 0; r < D; ++r)
 #pragma unroll
       for (int e = 0; e < D; ++e) acc[r] += v[r * D + e] * xv[e];
+  }
+}
+
+// Several waves per slice (the split kernels): part s of split_parts(D) of a
+// slice is the s-th share of its block slots, wave w takes parts w, w + waves,
+// ... and wave 0 adds the partial rows in a fixed order, whatever the
+// workgroup's size.  A slice then keeps several times the loads in flight, and
+// a matrix of a few thousand slices fills the chip (a wave per slice leaves one
+// or two waves per SIMD: Brick8 64x32x32, 1107 slices).  The values are read
+// through the caches: they stay in the last-level cache from one iteration to
+// the next, where streaming loads fetch them anew (the product alone, Q8
+// 512x256, 199 MB: 42 against 33 us).  Workgroup lb sweeps slices lb, lb + nlb,
+// ...; the partial rows are double-buffered in LDS, one workgroup barrier per
+// slice.  f(R, acc) is called by wave 0's lanes for their node rows R.
+__host__ __device__ constexpr int split_parts(int d) { return d == 2 ? 4 : 8; }
+struct SplitSlice {  // where workgroup lb starts: loaded before anything it waits for
+  int64_t sl, b0, b1;
+  int32_t R;
+};
+__device__ inline SplitSlice split_slice(int64_t sl, const BsellView& bs) {
+  SplitSlice s = {sl, 0, 0, -1};
+  if (sl < bs.nslices) {
+    s.b0 = bs.sptr[sl];
+    s.b1 = bs.sptr[sl + 1];
+    s.R = bs.perm[sl * 64 + (threadIdx.x & 63)];
+  }
+  return s;
+}
+template <int D, class X, class F>
+__device__ inline void for_rows_split(SplitSlice s, int nlb, int waves, const BsellView& bs,
+                                      const double* __restrict__ val,
+                                      const int32_t* __restrict__ bcol, const X x, F&& f) {
+  constexpr int P = split_parts(D), U = D == 2 ? 2 : 3;
+  __shared__ double sh_row[2][P][D][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  int buf = 0;
+  while (s.sl < bs.nslices) {
+    const int32_t w = int32_t(s.b1 - s.b0), R = s.R, Rn = R >= 0 ? R : 0;
+    for (int part = wave; part < P; part += waves) {
+      const int32_t j0 = w * part / P, cnt = w * (part + 1) / P - j0;
+      double acc[D];
+      if (bs.coff)
+        bsell_row<D, double, true, false, U, false>(bs, val, bcol, s.b0 + j0, cnt, lane, x, acc, Rn);
+      else
+        bsell_row<D, double, false, false, U, false>(bs, val, bcol, s.b0 + j0, cnt, lane, x, acc, 0);
+#pragma unroll
+      for (int r = 0; r < D; ++r) sh_row[buf][part][r][lane] = acc[r];
+    }
+    s = split_slice(s.sl + nlb, bs);
+    __syncthreads();
+    if (wave == 0 && R >= 0) {
+      double acc[D];
+#pragma unroll
+      for (int r = 0; r < D; ++r) {
+        double v[P];
+#pragma unroll
+        for (int k = 0; k < P; ++k) v[k] = sh_row[buf][k][r][lane];
+#pragma unroll
+        for (int k = P / 2; k > 0; k /= 2)
+#pragma unroll
+          for (int j = 0; j < k; ++j) v[j] = v[2 * j] + v[2 * j + 1];
+        acc[r] = v[0];
+      }
+      f(R, acc);
+    }
+    buf ^= 1;
   }
 }
 

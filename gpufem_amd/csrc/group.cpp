@@ -365,7 +365,7 @@ int gf_group_pcg(gf_ctx* ctx, gf_group* g, const double* b, double* x, const gf_
   gf_ell* m = g->ell;
   int st = ensure_plan(ctx, m);
   if (st) return st;
-  if (m->plan->variant < 0 && (st = tune_spmv(ctx, m, -1, nullptr, nullptr))) return st;
+  if ((st = choose_variant(ctx, m))) return st;
   if ((st = prepare_jacobi(ctx, m))) return st;
   if ((st = prepare_variant(ctx, m, group_variant(m)))) return st;
   // the ELL values unless the grouped kernels read the block-sliced copy

@@ -117,6 +117,13 @@ inline bool is_bsell_group_variant(int v) { return v == kBsell2G || v == kBsell3
 inline bool is_bsell_variant(int v) {
   return v == kBsell2 || v == kBsell3 || is_bsell_group_variant(v);
 }
+// The solver's own kernels over the block-sliced copy inside an iteration
+// (never a public variant number): several waves share a slice and a bounded
+// grid sweeps the slices (for_rows_split).
+enum IterVariant { kSplit2 = 11, kSplit3 = 12 };
+inline bool is_split_variant(int v) { return v == kSplit2 || v == kSplit3; }
+// what the last-level cache holds
+constexpr int64_t kCacheBytes = int64_t(256) << 20;
 // node columns: coln[i + j n] = col[i + d j n] / d for j < width / d
 hipError_t launch_build_coln(hipStream_t s, int64_t n, int32_t width, int d, const int32_t* col,
                              int32_t* coln);
@@ -171,12 +178,19 @@ hipError_t launch_bsell_to_ell(hipStream_t s, const BsellView& bs, int d, int64_
 constexpr int kMaxPcgBlocks = 2048;
 // SpMV workgroups of the slice-group variants (one partial p.q each)
 constexpr int kMaxSpmvBlocks = 65536;
+// most workgroups of the split kernels (each leaves a partial p.q that every
+// workgroup of the update adds); larger matrices take sweeps
+constexpr int kSplitBlocks = 4096;
 
 // workgroups of the standalone SpMV and the PCG kernels for n rows
 int spmv_blocks(int64_t n);
 // workgroups of the SpMV kernels of `variant`: one per four-slice group for
 // the slice-group variants, else `nblocks`
 int spmv_grid(int variant, const BsellView& bs, int nblocks);
+// the kernel that forms q = K p inside an iteration: the split kernels for the
+// slice-group variants while the block values (bslots block slots of
+// value_bytes each) stay in the last-level cache, else the variant itself
+int iter_variant(int variant, int64_t bslots, int64_t value_bytes);
 // bs: the block-sliced view (used by the kBsell variants only; may be null)
 hipError_t launch_spmv(hipStream_t s, int variant, int64_t n, const double* val,
                        const int32_t* col, const int32_t* rownnz, const double* x, double* y,
@@ -191,7 +205,8 @@ struct PcgState;  // device-resident scalars (solver.hip)
 struct PcgBuffers {
   int64_t n;
   int32_t width;
-  int variant;
+  int variant;       // products outside the iteration (launch_spmv)
+  int iter_variant;  // q = K p inside it; a split variant: the two-launch iteration
   const double* val;
   const int32_t* col;
   const int32_t* rownnz;
@@ -199,7 +214,7 @@ struct PcgBuffers {
   const double* b;
   double* x;
   double* r;
-  double* z;
+  double* z;  // z and p: component-major (c * nodes + node) in the two-launch iteration
   double* p;
   double* q;
   double* part1;  // per-SpMV-workgroup partials of p.q
@@ -217,23 +232,28 @@ hipError_t launch_pcg_iteration(hipStream_t s, const PcgBuffers& B, int parity);
 // the same, with events recorded around the SpMV kernel
 hipError_t launch_pcg_iteration_timed(hipStream_t s, const PcgBuffers& B, int parity,
                                       hipEvent_t spmv_start, hipEvent_t spmv_stop);
-// co-resident workgroups for the persistent kernel of this variant (0: unavailable)
+// after iterations, the next of which has this parity: the state they left
+hipError_t launch_pcg_check(hipStream_t s, const PcgBuffers& B, int parity);
+// co-resident workgroups for the persistent kernel of this (iteration) variant
+// (0: unavailable)
 int persistent_blocks(int variant, int num_cu);
 // nbar grid barriers of the persistent schedule on a cooperative grid of
 // nblocks workgroups; barrier_aborted reads whether a wait hit its spin limit
 hipError_t launch_barrier_probe(hipStream_t s, void* barrier, int nblocks, int nbar);
 int barrier_aborted(hipStream_t s, const void* barrier, int* aborted);
 // all remaining iterations in one cooperative launch
-hipError_t launch_pcg_persistent(hipStream_t s, const PcgBuffers& B, void* barrier);
+hipError_t launch_pcg_persistent(hipStream_t s, const PcgBuffers& B, void* barrier, int num_cu);
 // Host view of the scalar state.
 struct PcgHostState {
   int32_t it, done, status;
   int32_t x0_rejected;  // set by the host: a guarded initial guess was replaced by zero
-  double rr, bnorm2, rho;
+  double rr, bnorm2;
 };
 hipError_t read_pcg_state(hipStream_t s, const PcgBuffers& B, PcgHostState* h);
-// nrep launches of the iteration's SpMV kernel with the state forced live
-hipError_t launch_spmv_pq_repeat(hipStream_t s, const PcgBuffers& B, int nrep);
+// nrep launches of the iteration's SpMV kernel with the state forced live; with
+// `direction` each is followed by the direction pass where that is separate
+hipError_t launch_spmv_pq_repeat(hipStream_t s, const PcgBuffers& B, int nrep,
+                                 bool direction = false);
 // true residual ||b - K x|| / ||b|| into *out (device), deterministic
 hipError_t launch_true_residual(hipStream_t s, const PcgBuffers& B, double* out_dev);
 // *out_dev = 1/2 x.Kx - b.x (B.q is overwritten with K x)

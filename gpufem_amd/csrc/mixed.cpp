@@ -236,7 +236,6 @@ int run_mixed(gf_ctx* ctx, gf_ell* m, const gf_solve_opts& opts, PcgHostState* h
   h->status = hs.status;
   h->rr = hs.rr_true;
   h->bnorm2 = hs.bnorm2;
-  h->rho = 0.0;
   *refinements = hs.refinements;
   return GF_OK;
 }

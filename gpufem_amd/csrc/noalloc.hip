@@ -116,6 +116,7 @@ extern "C" int gf_pcg_noalloc(gf_ctx* ctx, gf_ell* m, const double* b, double* x
   B.n = n;
   B.width = m->width;
   B.variant = variant;
+  B.iter_variant = iter_variant(variant, m->bslots, sizeof(double));
   B.val = o.val;
   B.col = o.col;
   B.bs = o.bs;
@@ -130,8 +131,8 @@ extern "C" int gf_pcg_noalloc(gf_ctx* ctx, gf_ell* m, const double* b, double* x
   B.q = reinterpret_cast<double*>(base + 4 * kVecBytes);
   B.part1 = reinterpret_cast<double*>(base + kPart1Off);
   B.part2 = reinterpret_cast<double*>(base + kPart2Off);
-  B.nblocks = pcg_grid(variant, n, ctx->num_cu);
-  B.spmv_grid = spmv_grid(variant, o.bs, B.nblocks);
+  B.nblocks = pcg_grid(B.iter_variant, n, ctx->num_cu);
+  B.spmv_grid = spmv_grid(B.iter_variant, o.bs, B.nblocks);
   B.st = reinterpret_cast<PcgState*>(base + kStateOff);
   double* res = reinterpret_cast<double*>(base + kResOff);
 
@@ -145,6 +146,7 @@ extern "C" int gf_pcg_noalloc(gf_ctx* ctx, gf_ell* m, const double* b, double* x
     while (!h.done) {
       for (int it = 0; it < kChunk; ++it)
         GF_HIP_CHECK(ctx, launch_pcg_iteration(ctx->stream, B, it & 1));
+      GF_HIP_CHECK(ctx, launch_pcg_check(ctx->stream, B, 0));
       GF_HIP_CHECK(ctx, read_pcg_state(ctx->stream, B, &h));
     }
     total += h.it;

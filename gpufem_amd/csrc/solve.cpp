@@ -6,8 +6,8 @@
 // residual b - K x is then checked and PCG restarted from x while it exceeds
 // rtol.  The true residual at exit is always reported.  The
 // workspace (vectors, partials, scalar state, captured graphs) is cached on
-// the matrix; the SpMV variant is picked once per matrix by timing every
-// variant on the matrix itself.
+// the matrix; the SpMV variant is picked once per matrix, by its size or by
+// timing every variant on the matrix itself.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -54,6 +54,7 @@ hipError_t ensure_graph(gf_ctx* ctx, gf_ell* m, const PcgBuffers& B, int key) {
     e = launch_pcg_iteration(ctx->stream, B, it & 1);
     if (e != hipSuccess) break;
   }
+  if (e == hipSuccess) e = launch_pcg_check(ctx->stream, B, 0);
   hipError_t e2 = hipStreamEndCapture(ctx->stream, &g);
   if (e == hipSuccess) e = e2;
   if (e == hipSuccess) e = hipGraphInstantiate(&P->graph[key], g, nullptr, nullptr, 0);
@@ -89,9 +90,10 @@ int ensure_plan(gf_ctx* ctx, gf_ell* m) {
 
 // Fixes the variant and the PCG grid (the same grid for every schedule, so
 // all schedules give bitwise-identical results).
-int pcg_grid(int variant, int64_t n, int num_cu) {
+int pcg_grid(int iter_variant, int64_t n, int num_cu) {
   int nb = spmv_blocks(n);
-  const int pc = persistent_blocks(variant, num_cu);
+  // the split kernels' persistent solve plays the grid's workgroups in turn
+  const int pc = is_split_variant(iter_variant) ? nb : persistent_blocks(iter_variant, num_cu);
   if (pc > 0 && nb > pc) nb = pc;
   if (nb >= 8) nb &= ~7;
   return std::max(1, nb);
@@ -102,8 +104,9 @@ void set_variant(gf_ell* m, int variant) {
   if (P->variant == variant && P->nblocks > 0) return;
   drop_graphs(P);
   P->variant = variant;
-  P->persistent_ok = persistent_blocks(variant, P->num_cu) > 0;
-  P->nblocks = pcg_grid(variant, m->n, P->num_cu);
+  const int iter = iter_variant(variant, m->bslots, sizeof(double));
+  P->persistent_ok = persistent_blocks(iter, P->num_cu) > 0;
+  P->nblocks = pcg_grid(iter, m->n, P->num_cu);
 }
 
 // The node-block / block-sliced variants of the matrix's dimension, or -1
@@ -291,6 +294,7 @@ PcgBuffers make_buffers(gf_ell* m, const double* dinv) {
   B.n = m->n;
   B.width = m->width;
   B.variant = P->variant;
+  B.iter_variant = iter_variant(P->variant, m->bslots, sizeof(double));
   B.val = o.val;
   B.col = o.col;
   B.bs = o.bs;
@@ -305,9 +309,18 @@ PcgBuffers make_buffers(gf_ell* m, const double* dinv) {
   B.part1 = P->part1;
   B.part2 = P->part2;
   B.nblocks = P->nblocks;
-  B.spmv_grid = spmv_grid(P->variant, o.bs, P->nblocks);
+  B.spmv_grid = spmv_grid(B.iter_variant, o.bs, P->nblocks);
   B.st = P->st;
   return B;
+}
+
+// the slice-group variant of a matrix whose block-sliced copy (built) runs the
+// split kernels, or -1
+int cached_variant(const gf_ell* m) {
+  const int b = bsell_variant(m);
+  if (b < 0 || !m->d_bperm) return -1;
+  const int g = b == kBsell2 ? kBsell2G : kBsell3G;
+  return is_split_variant(iter_variant(g, m->bslots, sizeof(double))) ? g : -1;
 }
 
 int tune_spmv(gf_ctx* ctx, gf_ell* m, int force, double* ms_out, int* chosen) {
@@ -324,7 +337,7 @@ int tune_spmv(gf_ctx* ctx, gf_ell* m, int force, double* ms_out, int* chosen) {
     return GF_OK;
   }
   GF_HIP_CHECK(ctx, hipMemsetAsync(P->p, 0, size_t(m->n) * sizeof(double), ctx->stream));
-  const int reps = m->n > 200000 ? 10 : 30;
+  const int reps = m->n > 200000 ? 10 : 16;
   double best = 1e300;
   int best_v = kThreadU8;
   for (int v = 0; v < kNumSpmvVariants; ++v) {
@@ -335,9 +348,9 @@ int tune_spmv(gf_ctx* ctx, gf_ell* m, int force, double* ms_out, int* chosen) {
     if ((st = prepare_variant(ctx, m, v))) return st;
     set_variant(m, v);
     PcgBuffers B = make_buffers(m, nullptr);
-    GF_HIP_CHECK(ctx, launch_spmv_pq_repeat(ctx->stream, B, 2));
+    GF_HIP_CHECK(ctx, launch_spmv_pq_repeat(ctx->stream, B, 2, true));
     GF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_start, ctx->stream));
-    GF_HIP_CHECK(ctx, launch_spmv_pq_repeat(ctx->stream, B, reps));
+    GF_HIP_CHECK(ctx, launch_spmv_pq_repeat(ctx->stream, B, reps, true));
     GF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_stop, ctx->stream));
     GF_HIP_CHECK(ctx, hipEventSynchronize(ctx->ev_stop));
     float ms = 0.f;
@@ -352,6 +365,26 @@ int tune_spmv(gf_ctx* ctx, gf_ell* m, int force, double* ms_out, int* chosen) {
   set_variant(m, best_v);
   if (chosen) *chosen = best_v;
   return GF_OK;
+}
+
+// The variant of a solve whose caller chose none: the slice-group variant
+// untimed for a matrix that stays in the last-level cache, whose two-launch
+// iteration is the fastest on every size measured (Q4 64x32 to Brick20 24^3;
+// timing eleven variants took 12 ms of an 89 ms analysis of Q8 201x67), else
+// the fastest by measurement.
+int choose_variant(gf_ctx* ctx, gf_ell* m) {
+  int st = ensure_plan(ctx, m);
+  if (st || m->plan->variant >= 0) return st;
+  if (bsell_variant(m) >= 0) {
+    if ((st = ensure_bsell(ctx, m))) return st;
+    const int v = cached_variant(m);
+    if (v >= 0) {
+      if ((st = prepare_variant(ctx, m, v))) return st;
+      set_variant(m, v);
+      return GF_OK;
+    }
+  }
+  return tune_spmv(ctx, m, -1, nullptr, nullptr);
 }
 
 // Runs one right-hand side already placed in the plan's wb (and wx when
@@ -374,7 +407,7 @@ int run_pcg(gf_ctx* ctx, gf_ell* m, const PcgBuffers& B, int sched, int key, int
     if (!set_up) GF_HIP_CHECK(ctx, launch_pcg_setup(ctx->stream, B, use_x0, rtol, maxit - total));
     set_up = false;
     if (sched == GF_SCHED_PERSISTENT) {
-      GF_HIP_CHECK(ctx, launch_pcg_persistent(ctx->stream, B, P->barrier));
+      GF_HIP_CHECK(ctx, launch_pcg_persistent(ctx->stream, B, P->barrier, P->num_cu));
       GF_HIP_CHECK(ctx, read_pcg_state(ctx->stream, B, h));
       if (h->status == GF_ERR_HIP)
         return set_error(ctx, GF_ERR_HIP, "gf_pcg: grid barrier timed out in the persistent kernel");
@@ -387,6 +420,7 @@ int run_pcg(gf_ctx* ctx, gf_ell* m, const PcgBuffers& B, int sched, int key, int
         } else {
           for (int it = 0; it < kChunk; ++it)
             GF_HIP_CHECK(ctx, launch_pcg_iteration(ctx->stream, B, it & 1));
+          GF_HIP_CHECK(ctx, launch_pcg_check(ctx->stream, B, 0));
         }
         GF_HIP_CHECK(ctx, read_pcg_state(ctx->stream, B, h));
       }
@@ -484,7 +518,7 @@ int gf_pcg(gf_ctx* ctx, gf_ell* m, const double* b, double* x, int32_t nrhs,
   int st = ensure_plan(ctx, m);
   if (st) return st;
   gf_solve_plan* P = m->plan;
-  if (P->variant < 0 && (st = tune_spmv(ctx, m, -1, nullptr, nullptr))) return st;
+  if ((st = choose_variant(ctx, m))) return st;
   const int64_t n = m->n;
   const size_t vb = size_t(n) * sizeof(double);
   int sched = opts.schedule == GF_SCHED_AUTO ? GF_SCHED_GRAPH : opts.schedule;
@@ -693,7 +727,7 @@ int gf_profile_spmv(gf_ctx* ctx, gf_ell* m, int32_t nrep, double* ms_avg) {
   GF_HIP_CHECK(ctx, hipSetDevice(ctx->device));
   int st = ensure_plan(ctx, m);
   if (st) return st;
-  if (m->plan->variant < 0 && (st = tune_spmv(ctx, m, -1, nullptr, nullptr))) return st;
+  if ((st = choose_variant(ctx, m))) return st;
   if ((st = prepare_variant(ctx, m, m->plan->variant))) return st;
   PcgBuffers B = make_buffers(m, nullptr);
   GF_HIP_CHECK(ctx, hipMemsetAsync(m->plan->p, 0, size_t(m->n) * sizeof(double), ctx->stream));
@@ -716,7 +750,7 @@ int gf_profile_barrier(gf_ctx* ctx, gf_ell* m, int32_t nbar, double* us_per_barr
   int st = ensure_plan(ctx, m);
   if (st) return st;
   gf_solve_plan* P = m->plan;
-  if (P->variant < 0 && (st = tune_spmv(ctx, m, -1, nullptr, nullptr))) return st;
+  if ((st = choose_variant(ctx, m))) return st;
   const int nb = persistent_blocks(P->variant, P->num_cu);
   if (nb < 1)
     return set_error(ctx, GF_ERR_UNSUPPORTED, "gf_profile_barrier: no persistent grid for this matrix");
@@ -746,7 +780,7 @@ int gf_profile_pcg(gf_ctx* ctx, gf_ell* m, const double* b, int32_t iters, doubl
   int st = ensure_plan(ctx, m);
   if (st) return st;
   gf_solve_plan* P = m->plan;
-  if (P->variant < 0 && (st = tune_spmv(ctx, m, -1, nullptr, nullptr))) return st;
+  if ((st = choose_variant(ctx, m))) return st;
   if ((st = prepare_jacobi(ctx, m))) return st;
   if ((st = prepare_variant(ctx, m, P->variant))) return st;
   GF_HIP_CHECK(ctx, hipMemcpyAsync(P->wb, b, size_t(m->n) * sizeof(double),
@@ -779,6 +813,7 @@ int gf_profile_pcg(gf_ctx* ctx, gf_ell* m, const double* b, int32_t iters, doubl
     }
     done += c;
   }
+  GF_HIP_CHECK(ctx, launch_pcg_check(ctx->stream, B, iters & 1));
   GF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_stop, ctx->stream));
   GF_HIP_CHECK(ctx, hipEventSynchronize(ctx->ev_stop));
   float total = 0.f;

@@ -32,9 +32,11 @@ namespace gf {
 void release_solve_plan(gf_ell* m);
 int ensure_plan(gf_ctx* ctx, gf_ell* m);
 void set_variant(gf_ell* m, int variant);
-// workgroups of the PCG kernels for this variant and size (the grid every
+// workgroups of the PCG kernels for this iteration variant and size (the grid every
 // schedule uses, so all give bitwise-identical results)
-int pcg_grid(int variant, int64_t n, int num_cu);
+int pcg_grid(int iter_variant, int64_t n, int num_cu);
+// fixes the variant of a matrix never tuned
+int choose_variant(gf_ctx* ctx, gf_ell* m);
 int tune_spmv(gf_ctx* ctx, gf_ell* m, int force, double* ms_out, int* chosen);
 PcgBuffers make_buffers(gf_ell* m, const double* dinv);
 // arrays the SpMV variant reads: the ELL arrays, the node columns (kNode) or

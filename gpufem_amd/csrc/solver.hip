@@ -21,11 +21,15 @@
 //   kBsell2G/3G      the same with one workgroup per four-slice group (one
 //                    sweep; the dispatcher balances unequal slices).
 //
+// Inside an iteration the slice-group variants run the split kernels while the
+// matrix stays in the last-level cache (iter_variant).
+//
 // CG schedules: three launches per iteration (k_spmv_pq, k_update,
-// k_direction) with all scalars in a device PcgState, so the host can
+// k_direction), or two (k_split_product, k_split_update; k_split_check after a
+// chunk of them), with all scalars in a device PcgState, so the host can
 // enqueue or graph-replay chunks of iterations; or one cooperative
-// persistent kernel (k_pcg_persistent) with three grid barriers per
-// iteration.  Every block reduces the per-block partials in the same fixed
+// persistent kernel (k_pcg_persistent, k_split_persistent) with a grid barrier
+// after each of those steps.  Every block reduces the per-block partials in the same fixed
 // order, so all blocks take the same convergence decision and results are
 // bitwise reproducible for a given matrix and variant.  The SpMV kernel may
 // run on a grid of its own (the slice-group variants): k_update reduces its
@@ -33,6 +37,8 @@
 // SpMV workgroups in turn.  No workgroup waits on another inside a kernel
 // but the persistent one: on gfx950 an agent-scope release writes back the
 // XCD's L2, far too costly once per workgroup per SpMV.
+#include <algorithm>
+
 #include "device_common.hpp"
 #include "gf_internal.hpp"
 #include "launch.hpp"
@@ -44,7 +50,10 @@ struct PcgState {
   double rr;      // r.r after the last update
   double bnorm2;  // b.b
   double rtol2;   // rtol^2
-  double spare;
+  // two-launch iteration: iterations done, by parity (a launch of parity P
+  // reads itv[P] and writes itv[P ^ 1], rho[P] likewise: no workgroup of it
+  // can see the value it leaves); it: the count at the last check
+  int32_t itv[2];
   int32_t it;
   int32_t done;
   int32_t status;
@@ -207,7 +216,186 @@ __device__ inline void phase_direction(const PcgBuffers& B, double beta) {
   for_my_rows(B.n, [&](int64_t i) { B.p[i] = B.z[i] + beta * B.p[i]; });
 }
 
+// ---------------------------------------------------------------------------
+// The two-launch iteration (split variants).  The direction is never stored on
+// its own: the product forms p_k = z_k + beta_k p_{k-1} in its gathers and the
+// update forms it again for its own rows, which then hold (z_{k+1}, p_k) in
+// place; beta comes from the same sums, in the same order and with the same
+// rounding as in a direction pass of its own.  An iteration, with the split
+// product, against the three launches before: Brick8 64x32x32 37.0 / 43.6 us,
+// Q8 512x256 53.6 / 66.0, Q8 201x67 13.2 / 18.9, Q4 64x32 9.8 / 13.5, Brick20
+// 24^3 61 / 64.  A matrix that streams from memory keeps the three launches:
+// there the second gather costs 23 us a product (Brick8 96^3), more than the
+// direction pass it saves.
+// ---------------------------------------------------------------------------
+// The product's slices from `first` on in steps of nlb, `waves` waves; wave 0's
+// lanes return their part of p.q
+template <int D>
+__device__ inline double phase_split(const PcgBuffers& B, SplitSlice first, int nlb, int waves,
+                                     double beta) {
+  double pq = 0.0;
+  const LazyDirection<D> p{B.z, B.p, B.n / D, beta};
+  double* __restrict__ q = B.q;
+  for_rows_split<D>(first, nlb, waves, B.bs, B.val, B.col, p, [&](int32_t R, const double* acc) {
+#pragma unroll
+    for (int r = 0; r < D; ++r) {
+      q[int64_t(D) * R + r] = acc[r];
+      pq += p.at(R, r) * acc[r];
+    }
+  });
+  return pq;
+}
+
+// the sum over wave 0's lanes, written by lane 0
+__device__ inline void store_wave_sum(double v, double* out) {
+  if (threadIdx.x >= 64) return;
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  if (threadIdx.x == 0) *out = v;
+}
+
+// kRows rows of a thread at a time: the loads of the first ones are issued
+// before the scalars of the iteration are known (their latency and the
+// reduction's overlap).  Row i = D node + e of the solver's vectors is entry
+// e * nodes + node of z and p.
+constexpr int kRows = 4;
+struct SplitRows {
+  double x[kRows], z[kRows], p[kRows], r[kRows], q[kRows], d[kRows];
+};
+template <int D>
+__device__ inline int64_t lazy_index(const PcgBuffers& B, int64_t i) {
+  const uint32_t node = uint32_t(i) / D, e = uint32_t(i) - node * D;
+  return int64_t(e) * (B.n / D) + node;
+}
+template <int D>
+__device__ inline void split_load(const PcgBuffers& B, int64_t base, int64_t stride, SplitRows* v) {
+#pragma unroll
+  for (int u = 0; u < kRows; ++u) {
+    const int64_t i = base + u * stride;
+    if (i < B.n) {
+      const int64_t k = lazy_index<D>(B, i);
+      v->z[u] = B.z[k];
+      v->p[u] = B.p[k];
+      v->x[u] = B.x[i];
+      v->r[u] = B.r[i];
+      v->q[u] = B.q[i];
+      v->d[u] = B.dinv ? B.dinv[i] : 1.0;
+    }
+  }
+}
+// x += alpha p; r -= alpha q; z = M^-1 r over the rows of logical workgroup lb
+// (the first ones already in v); the sums r.z and r.r of it to part2[slot]
+template <int D>
+__device__ inline void phase_split_update(const PcgBuffers& B, int lb, int slot, double alpha,
+                                          double beta, SplitRows& v, double* sh) {
+  double rz = 0.0, rr = 0.0;
+  const int64_t stride = int64_t(B.nblocks) * kNT;
+  for (int64_t base = int64_t(lb) * kNT + threadIdx.x;;) {
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+      const int64_t i = base + u * stride;
+      if (i < B.n) {
+        const int64_t k = lazy_index<D>(B, i);
+        const double pi = v.z[u] + beta * v.p[u];
+        const double ri = v.r[u] - alpha * v.q[u];
+        const double zi = B.dinv ? v.d[u] * ri : ri;
+        B.x[i] = v.x[u] + alpha * pi;
+        B.r[i] = ri;
+        B.z[k] = zi;
+        B.p[k] = pi;
+        rz += ri * zi;
+        rr += ri * ri;
+      }
+    }
+    base += kRows * stride;
+    if (base >= B.n) break;
+    split_load<D>(B, base, stride, &v);
+  }
+  block_sum2(&rz, &rr, sh);
+  if (threadIdx.x == 0) {
+    B.part2[slot] = rz;
+    B.part2[B.nblocks + slot] = rr;
+  }
+}
+
+// Whether iteration `it` runs, from the residual sum every workgroup forms in
+// the same order; `lead` sets the state when it does not.
+__device__ inline bool split_goes_on(const PcgBuffers& B, int it, double rr, bool lead) {
+  PcgState* st = B.st;
+  if (!(rr <= st->rtol2 * st->bnorm2) && it < st->maxit) return true;
+  if (lead) {
+    st->rr = rr;
+    st->it = it;
+    st->done = 1;
+  }
+  return false;
+}
+__device__ inline void split_breakdown(const PcgBuffers& B, int it, bool lead) {
+  if (!lead) return;
+  B.st->it = it;
+  B.st->status = GF_ERR_BREAKDOWN;
+  B.st->done = 1;
+}
+__device__ inline double split_beta(int it, double rz, double rz_old) {
+  return it > 0 ? rz / rz_old : 0.0;
+}
+
+// First launch: the stopping test, beta and q = K p.  `done` changes inside a
+// launch only when none of its workgroups writes a vector, so one that starts
+// late and reads it set leaves nothing undone.
+// Every load that waits for nothing is issued before the first wait (the flag
+// included: a finished state costs the loads of one launch).
+template <int D>
+__global__ __launch_bounds__(64 * split_parts(D), D == 2 ? 6 : 4) void k_split_product(
+    PcgBuffers B, int parity) {
+  PcgState* st = B.st;
+  __shared__ double sh[2 * (kNT / 64)];
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  const SplitSlice first = split_slice(logical_block(), B.bs);
+  const int it = st->itv[parity], done = st->done;
+  const double rz_old = st->rho[parity ^ 1];
+  double rz, rr;
+  reduce_partials2(B.part2, B.part2 + B.nblocks, B.nblocks, &rz, &rr, sh);
+  if (done || !split_goes_on(B, it, rr, lead)) return;
+  if (lead) st->rho[parity] = rz;
+  const double beta = split_beta(it, rz, rz_old);
+  store_wave_sum(phase_split<D>(B, first, gridDim.x, split_parts(D), beta), B.part1 + blockIdx.x);
+}
+
+// Second launch: alpha and the vector updates.
+template <int D>
+__global__ __launch_bounds__(kNT) void k_split_update(PcgBuffers B, int parity) {
+  PcgState* st = B.st;
+  __shared__ double sh[2 * (kNT / 64)];
+  SplitRows v;
+  const int lb = logical_block();
+  split_load<D>(B, int64_t(lb) * kNT + threadIdx.x, int64_t(B.nblocks) * kNT, &v);
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  const int it = st->itv[parity], done = st->done;
+  const double rho = st->rho[parity], beta = split_beta(it, rho, st->rho[parity ^ 1]);
+  const double pq = reduce_partials(B.part1, B.spmv_grid, sh);
+  if (done) return;
+  if (!(pq > 0.0)) return split_breakdown(B, it, lead);
+  phase_split_update<D>(B, lb, blockIdx.x, rho / pq, beta, v, sh);
+  if (lead) st->itv[parity ^ 1] = it + 1;
+}
+
+// The state the host reads: the last residual checked as the next iteration
+// (of this parity) would check it.
+__global__ __launch_bounds__(kNT) void k_split_check(PcgBuffers B, int parity) {
+  if (B.st->done) return;
+  __shared__ double sh[kNT / 64];
+  const double rr = reduce_partials(B.part2 + B.nblocks, B.nblocks, sh);
+  if (threadIdx.x == 0) {
+    PcgState* st = B.st;
+    st->rr = rr;
+    st->it = st->itv[parity];
+    (void)split_goes_on(B, st->it, rr, true);
+  }
+}
+
 // r = b - q (use_x0) or x = 0, r = b; z = M^-1 r; p = z; partials r.z, r.r, b.b
+// (SOA > 1: z in the two-launch iteration's order, its p_old = 0)
+template <int SOA>
 __global__ __launch_bounds__(kNT) void k_pcg_init(PcgBuffers B, int use_x0) {
   __shared__ double sh[kNT / 64];
   double rz = 0, rr = 0, bb = 0;
@@ -222,8 +410,14 @@ __global__ __launch_bounds__(kNT) void k_pcg_init(PcgBuffers B, int use_x0) {
     }
     const double zi = B.dinv ? B.dinv[i] * ri : ri;
     B.r[i] = ri;
-    B.z[i] = zi;
-    B.p[i] = zi;
+    if constexpr (SOA > 1) {
+      const int64_t k = lazy_index<SOA>(B, i);
+      B.z[k] = zi;
+      B.p[k] = 0.0;
+    } else {
+      B.z[i] = zi;
+      B.p[i] = zi;
+    }
     rz += ri * zi;
     rr += ri * ri;
     bb += bi * bi;
@@ -251,7 +445,7 @@ __global__ __launch_bounds__(kNT) void k_pcg_init_finish(PcgBuffers B, int nb, d
     st->rr = rr;
     st->bnorm2 = bb;
     st->rtol2 = rtol2;
-    st->it = 0;
+    st->itv[0] = st->itv[1] = st->it = 0;
     st->status = GF_OK;
     st->maxit = maxit;
     st->done = (rr <= rtol2 * bb) || maxit <= 0;
@@ -404,8 +598,54 @@ __global__ __launch_bounds__(kNT) void k_pcg_persistent(PcgBuffers B, GridBarrie
   }
 }
 
+// The two-launch iteration the same way, two grid barriers each.
+template <int D>
+__global__ __launch_bounds__(kNT) void k_split_persistent(PcgBuffers B, GridBarrier* bar) {
+  __shared__ double sh[2 * (kNT / 64)];
+  __shared__ int s_flag;
+  PcgState* st = B.st;
+  if (st->done) return;  // read before any block can change it (it only changes at exit)
+  if (threadIdx.x == 0) s_flag = 0;
+  __syncthreads();
+  const int nlb = B.spmv_grid;
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  double rho = 0.0;
+  for (int it = 0;; ++it) {
+    double rz, rr;
+    reduce_partials2(B.part2, B.part2 + B.nblocks, B.nblocks, &rz, &rr, sh);
+    if (!split_goes_on(B, it, rr, lead)) break;
+    const double beta = split_beta(it, rz, rho);
+    rho = rz;
+    // the product's logical workgroups j (same slices, same partial slots)
+    for (int j = blockIdx.x; j < nlb; j += gridDim.x) {
+      store_wave_sum(
+          phase_split<D>(B, split_slice(xcd_block(j, nlb), B.bs), nlb, kNT / 64, beta),
+          B.part1 + j);
+      __syncthreads();  // the next slices' partial rows
+    }
+    if (!grid_barrier(bar, &s_flag)) break;
+    const double pq = reduce_partials(B.part1, nlb, sh);
+    if (!(pq > 0.0)) {
+      split_breakdown(B, it, lead);
+      break;
+    }
+    // the update's logical workgroups likewise
+    for (int j = blockIdx.x; j < B.nblocks; j += gridDim.x) {
+      const int lb = xcd_block(j, B.nblocks);
+      SplitRows v;
+      split_load<D>(B, int64_t(lb) * kNT + threadIdx.x, int64_t(B.nblocks) * kNT, &v);
+      phase_split_update<D>(B, lb, j, rho / pq, beta, v, sh);
+    }
+    if (!grid_barrier(bar, &s_flag)) break;
+  }
+  if (lead && s_flag) {
+    st->status = GF_ERR_HIP;
+    st->done = 1;
+  }
+}
+
 // nbar grid barriers and nothing else: the synchronisation cost of the
-// persistent schedule (three per iteration) on its own grid
+// persistent schedule (two or three per iteration) on its own grid
 __global__ __launch_bounds__(kNT) void k_barrier_probe(GridBarrier* bar, int nbar) {
   __shared__ int s_flag;
   for (int k = 0; k < nbar; ++k)
@@ -473,10 +713,17 @@ __global__ __launch_bounds__(kNT) void k_energy_finish(PcgBuffers B, int nb, dou
   if (threadIdx.x == 0) out[0] = 0.5 * xq - xb;
 }
 
+// a state in which products and direction passes run whatever the partials hold
 __global__ void k_state_live(PcgState* st) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     st->done = 0;
     st->status = GF_OK;
+    st->itv[0] = 0;
+    st->maxit = INT32_MAX;
+    st->it = 0;
+    st->rho[0] = 1.0;
+    st->bnorm2 = 1.0;
+    st->rtol2 = -INFINITY;
   }
 }
 
@@ -550,7 +797,21 @@ hipError_t launch_bsell_to_ell(hipStream_t s, const BsellView& bs, int d, int64_
   return hipGetLastError();
 }
 
+int iter_variant(int variant, int64_t bslots, int64_t value_bytes) {
+  if (!is_bsell_group_variant(variant)) return variant;
+  const int d = variant == kBsell2G ? 2 : 3;
+  if (bslots * 64 * d * d * value_bytes > kCacheBytes) return variant;
+  return d == 2 ? kSplit2 : kSplit3;
+}
+
 int spmv_grid(int variant, const BsellView& bs, int nblocks) {
+  if (is_split_variant(variant)) {
+    // sweeps of equal size over at most kSplitBlocks workgroups
+    const int64_t sweeps = std::max<int64_t>(1, (bs.nslices + kSplitBlocks - 1) / kSplitBlocks);
+    int64_t nb = (bs.nslices + sweeps - 1) / sweeps;
+    if (nb >= 8) nb = (nb + 7) & ~int64_t(7);  // the XCD remap needs a multiple of 8
+    return int(std::max<int64_t>(1, nb));
+  }
   if (!is_bsell_group_variant(variant)) return nblocks;
   int64_t nb = (bs.nslices + kNT / 64 - 1) / (kNT / 64);
   nb = (nb + 7) & ~int64_t(7);  // the XCD remap needs a multiple of 8
@@ -589,34 +850,67 @@ hipError_t launch_pcg_setup(hipStream_t s, const PcgBuffers& B, int use_x0, doub
     e = launch_spmv(s, B.variant, B.n, B.val, B.col, B.rownnz, B.x, B.q, 1, &B.bs);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(k_pcg_init, dim3(B.nblocks), dim3(kNT), 0, s, B, use_x0);
+  if (B.iter_variant == kSplit2)
+    hipLaunchKernelGGL(k_pcg_init<2>, dim3(B.nblocks), dim3(kNT), 0, s, B, use_x0);
+  else if (B.iter_variant == kSplit3)
+    hipLaunchKernelGGL(k_pcg_init<3>, dim3(B.nblocks), dim3(kNT), 0, s, B, use_x0);
+  else
+    hipLaunchKernelGGL(k_pcg_init<1>, dim3(B.nblocks), dim3(kNT), 0, s, B, use_x0);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   hipLaunchKernelGGL(k_pcg_init_finish, dim3(1), dim3(kNT), 0, s, B, B.nblocks, rtol * rtol,
                      maxit);
   return hipGetLastError();
 }
 
+namespace {
+// the product of an iteration
+hipError_t launch_product(hipStream_t s, const PcgBuffers& B, int parity) {
+  const dim3 g(B.spmv_grid);
+  if (B.iter_variant == kSplit2) {
+    hipLaunchKernelGGL(k_split_product<2>, g, dim3(64 * split_parts(2)), 0, s, B, parity);
+  } else if (B.iter_variant == kSplit3) {
+    hipLaunchKernelGGL(k_split_product<3>, g, dim3(64 * split_parts(3)), 0, s, B, parity);
+  } else {
+    GF_DISPATCH_VARIANT(B.iter_variant, k_spmv_pq, g, s, B);
+  }
+  return hipGetLastError();
+}
+// and its vector updates
+hipError_t launch_updates(hipStream_t s, const PcgBuffers& B, int parity) {
+  const dim3 g(B.nblocks), blk(kNT);
+  if (B.iter_variant == kSplit2) {
+    hipLaunchKernelGGL(k_split_update<2>, g, blk, 0, s, B, parity);
+    return hipGetLastError();
+  }
+  if (B.iter_variant == kSplit3) {
+    hipLaunchKernelGGL(k_split_update<3>, g, blk, 0, s, B, parity);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL(k_update, g, blk, 0, s, B, parity);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_direction, g, blk, 0, s, B, parity);
+  return hipGetLastError();
+}
+}  // namespace
+
 hipError_t launch_pcg_iteration(hipStream_t s, const PcgBuffers& B, int parity) {
-  hipError_t e;
-  GF_DISPATCH_VARIANT(B.variant, k_spmv_pq, dim3(B.spmv_grid), s, B);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_update, dim3(B.nblocks), dim3(kNT), 0, s, B, parity);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_direction, dim3(B.nblocks), dim3(kNT), 0, s, B, parity);
+  const hipError_t e = launch_product(s, B, parity);
+  return e != hipSuccess ? e : launch_updates(s, B, parity);
+}
+
+hipError_t launch_pcg_check(hipStream_t s, const PcgBuffers& B, int parity) {
+  if (!is_split_variant(B.iter_variant)) return hipSuccess;  // the direction pass checks
+  hipLaunchKernelGGL(k_split_check, dim3(1), dim3(kNT), 0, s, B, parity);
   return hipGetLastError();
 }
 
 hipError_t launch_pcg_iteration_timed(hipStream_t s, const PcgBuffers& B, int parity,
                                       hipEvent_t spmv_start, hipEvent_t spmv_stop) {
   hipError_t e = hipEventRecord(spmv_start, s);
-  if (e != hipSuccess) return e;
-  GF_DISPATCH_VARIANT(B.variant, k_spmv_pq, dim3(B.spmv_grid), s, B);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  if ((e = hipEventRecord(spmv_stop, s)) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_update, dim3(B.nblocks), dim3(kNT), 0, s, B, parity);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_direction, dim3(B.nblocks), dim3(kNT), 0, s, B, parity);
-  return hipGetLastError();
+  if (e == hipSuccess) e = launch_product(s, B, parity);
+  if (e == hipSuccess) e = hipEventRecord(spmv_stop, s);
+  return e != hipSuccess ? e : launch_updates(s, B, parity);
 }
 
 int persistent_blocks(int variant, int num_cu) {
@@ -634,6 +928,8 @@ int persistent_blocks(int variant, int num_cu) {
     case kBsell3: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pcg_persistent<kBsell3>, kNT, 0); break;
     case kBsell2G: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pcg_persistent<kBsell2G>, kNT, 0); break;
     case kBsell3G: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pcg_persistent<kBsell3G>, kNT, 0); break;
+    case kSplit2: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_split_persistent<2>, kNT, 0); break;
+    case kSplit3: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_split_persistent<3>, kNT, 0); break;
     default: break;
   }
   if (e != hipSuccess || per_cu < 1) return 0;
@@ -643,15 +939,24 @@ int persistent_blocks(int variant, int num_cu) {
   return int(nb);
 }
 
-hipError_t launch_pcg_persistent(hipStream_t s, const PcgBuffers& B, void* barrier) {
+hipError_t launch_pcg_persistent(hipStream_t s, const PcgBuffers& B, void* barrier, int num_cu) {
   GridBarrier* bar = static_cast<GridBarrier*>(barrier);
   hipLaunchKernelGGL(k_barrier_reset, dim3(1), dim3(64), 0, s, bar);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   PcgBuffers Bc = B;
   void* args[] = {&Bc, &bar};
-  const dim3 g(B.nblocks), blk(kNT);
-  switch (B.variant) {
+  // the split kernels play the logical workgroups of both steps in turn; the
+  // others' vector steps take exactly the grid of the kernel schedule
+  int nb = B.nblocks;
+  if (is_split_variant(B.iter_variant)) {
+    nb = std::min(std::max(B.nblocks, B.spmv_grid), persistent_blocks(B.iter_variant, num_cu));
+    if (nb < 1) return hipErrorInvalidConfiguration;
+  }
+  const dim3 g(nb), blk(kNT);
+  switch (B.iter_variant) {
+    case kSplit2: return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(k_split_persistent<2>), g, blk, args, 0, s);
+    case kSplit3: return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(k_split_persistent<3>), g, blk, args, 0, s);
     case kThreadU1: return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(k_pcg_persistent<kThreadU1>), g, blk, args, 0, s);
     case kThreadU4: return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(k_pcg_persistent<kThreadU4>), g, blk, args, 0, s);
     case kThreadU8: return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(k_pcg_persistent<kThreadU8>), g, blk, args, 0, s);
@@ -696,16 +1001,18 @@ hipError_t read_pcg_state(hipStream_t s, const PcgBuffers& B, PcgHostState* h) {
   h->status = st.status;
   h->rr = st.rr;
   h->bnorm2 = st.bnorm2;
-  h->rho = st.rho[st.it & 1];
   return hipSuccess;
 }
 
-hipError_t launch_spmv_pq_repeat(hipStream_t s, const PcgBuffers& B, int nrep) {
+hipError_t launch_spmv_pq_repeat(hipStream_t s, const PcgBuffers& B, int nrep, bool direction) {
   hipLaunchKernelGGL(k_state_live, dim3(1), dim3(64), 0, s, B.st);
   hipError_t e = hipGetLastError();
   for (int i = 0; i < nrep && e == hipSuccess; ++i) {
-    GF_DISPATCH_VARIANT(B.variant, k_spmv_pq, dim3(B.spmv_grid), s, B);
-    e = hipGetLastError();
+    e = launch_product(s, B, 0);
+    if (e == hipSuccess && direction && !is_split_variant(B.iter_variant)) {
+      hipLaunchKernelGGL(k_direction, dim3(B.nblocks), dim3(kNT), 0, s, B, 0);
+      e = hipGetLastError();
+    }
   }
   return e;
 }

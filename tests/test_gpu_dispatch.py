@@ -5,6 +5,7 @@ import pytest
 
 import gpufem_amd as gf
 import oracle as O
+from gpufem_amd import problems as P
 
 pytestmark = pytest.mark.gpu
 
@@ -31,3 +32,59 @@ def test_untimed_assembly_kernel(gpu_ctx, t, nx, ny, nz, want):
     Ko, _ = O.assemble(g.dim, ng, conn, coords, 210000.0, 0.3, skip_zero=False)
     ov = Ko.export(Ko.max_rownnz())[0]
     assert np.abs(val - ov).max() <= 1e-12 * np.abs(ov).max()
+
+
+def assembled(ctx, t, nx, ny, nz):
+    p = P.structured(t, nx, ny, nz)
+    mesh = ctx.upload_mesh(p.elem_type, p.ngauss, p.conn, p.coords, p.E, p.nu)
+    K = ctx.symbolic(mesh)
+    ctx.assemble(mesh, K)
+    ctx.apply_penalty(K, p.fixed_dofs)
+    return p, K
+
+
+@pytest.mark.parametrize("t,nx,ny,nz", [
+    (gf.GF_Q4, 1, 1, 0), (gf.GF_Q4, 7, 7, 0), (gf.GF_Q4, 20, 2, 0),      # 4, 64 and 63 nodes
+    (gf.GF_Q8, 33, 9, 0), (gf.GF_BRICK8, 1, 1, 1), (gf.GF_BRICK8, 15, 7, 7),
+    (gf.GF_BRICK20, 5, 4, 3), (gf.GF_Q4, 520, 519, 0)])                  # the last: two sweeps
+def test_two_launch_iteration(gpu_ctx, t, nx, ny, nz):
+    """A solve whose caller chose no variant takes the split kernels; its
+    answer is the thread-per-row solve's at the same tolerance, preconditioned
+    and not, and its schedules agree bitwise."""
+    p, K = assembled(gpu_ctx, t, nx, ny, nz)
+    _, R = assembled(gpu_ctx, t, nx, ny, nz)
+    gpu_ctx.tune(R, 0)
+    big = p.ndof > 100000
+    for kw in ([dict()] if big else [dict(), dict(precond=gf.GF_PRECOND_NONE, verify=0)]):
+        plain = "precond" in kw
+        # without a preconditioner the penalty rows keep plain CG from
+        # converging: a fixed number of iterations is compared instead
+        opts = dict(kw, rtol=1e-4 if big else (0.0 if plain else 1e-10), raise_on_fail=not plain)
+        if plain:
+            opts.update(maxit=3)
+        x, s = gpu_ctx.pcg(K, p.f, **opts)
+        xr, sr = gpu_ctx.pcg(R, p.f, **opts)
+        assert abs(s.iterations - sr.iterations) <= 2 + sr.iterations // 100
+        # the same iterates to rounding; near the tolerance, to it times the
+        # condition of these meshes (below 1e6 for the converged ones)
+        assert np.linalg.norm(x - xr) <= (1e-4 if big else 1e-9) * np.linalg.norm(xr)
+        if not big:
+            for sched in (gf.GF_SCHED_KERNELS, gf.GF_SCHED_PERSISTENT):
+                xs, ss = gpu_ctx.pcg(K, p.f, schedule=sched, **opts)
+                assert ss.iterations == s.iterations and np.array_equal(xs, x)
+
+
+def test_two_launch_iteration_breakdown(gpu_ctx):
+    """A negative definite matrix breaks down at the first iteration and zero
+    right-hand sides stop at none, on every schedule."""
+    g = gf.Grid(gf.GF_Q4, 9, 5)
+    conn, coords = g.fill()
+    mesh = gpu_ctx.upload_mesh(gf.GF_Q4, 2, conn, coords, -1.0, 0.3)
+    K = gpu_ctx.symbolic(mesh)
+    gpu_ctx.assemble(mesh, K)
+    f = np.random.default_rng(0).normal(size=g.ndof)
+    for sched in (gf.GF_SCHED_KERNELS, gf.GF_SCHED_GRAPH, gf.GF_SCHED_PERSISTENT):
+        x, s = gpu_ctx.pcg(K, f, schedule=sched, precond=gf.GF_PRECOND_NONE, raise_on_fail=False)
+        assert s.code == gf.GF_ERR_BREAKDOWN and s.iterations == 0
+        x, s = gpu_ctx.pcg(K, 0.0 * f, schedule=sched)
+        assert s.converged and s.iterations == 0 and not x.any()
