@@ -436,6 +436,25 @@ __device__ inline void for_rows_split(SplitSlice s, int nlb, int waves, const Bs
   }
 }
 
+// the sum over wave 0's lanes, written by lane 0
+__device__ inline void store_wave_sum(double v, double* out) {
+  if (threadIdx.x >= 64) return;
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  if (threadIdx.x == 0) *out = v;
+}
+
+// beta of iteration `it` from r.z now and one iteration before
+__device__ inline double split_beta(int it, double rz, double rz_old) {
+  return it > 0 ? rz / rz_old : 0.0;
+}
+
+// where row i = D node + e of n rows lies in a component-major vector
+template <int D>
+__device__ inline int64_t lazy_index(int64_t i, int64_t n) {
+  const uint32_t node = uint32_t(i) / D, e = uint32_t(i) - node * D;
+  return int64_t(e) * (n / D) + node;
+}
+
 // Calls f(i, (K x)_i) for every row of logical workgroup lb of nlb, with
 // the SpMV variant V (thread per row with 1/4/8 slots in flight, 2/4 waves
 // sharing a tile of rows, node blocks, block-sliced slices).  Every thread of

@@ -31,6 +31,12 @@ struct gf_group {
   int64_t *d_sg_ptr = nullptr, *d_sg_s0 = nullptr, *d_sg_s1 = nullptr;
   int32_t* d_sg_mesh = nullptr;
   double* part_sg = nullptr;
+  // two-launch iteration (built with the slice groups when the copy stays in
+  // the last-level cache)
+  bool split = false;
+  double* split_buf = nullptr;    // z [n], part_sl [nslices], rho2 [2 nmesh]
+  int64_t* d_sl_ptr = nullptr;
+  int32_t* d_sl_mesh = nullptr;   // sl_mesh [nslices], it2 [2 nmesh]
   double* per_mesh = nullptr;   // rho, alpha, beta, rr, bb, pen, res: 7 * nmesh
   int32_t* per_mesh_i = nullptr;  // it, done, status: 3 * nmesh
   gf::GroupState* st = nullptr;
@@ -70,6 +76,9 @@ void group_release(gf_group* g) {
   dfree(g->d_sg_s1);
   dfree(g->d_sg_mesh);
   dfree(g->part_sg);
+  dfree(g->split_buf);
+  dfree(g->d_sl_ptr);
+  dfree(g->d_sl_mesh);
   dfree(g->st);
   if (g->ell) gf_ell_free(g->ell);
   if (g->mesh) gf_mesh_free(g->mesh);
@@ -113,6 +122,20 @@ int ensure_slice_groups(gf_ctx* ctx, gf_group* g) {
   if (e == hipSuccess) e = hipMalloc(&g->d_sg_s1, ns * 8);
   if (e == hipSuccess) e = hipMalloc(&g->d_sg_mesh, ns * 4);
   if (e == hipSuccess) e = hipMalloc(&g->part_sg, ns * 8);
+  // the two-launch iteration's arrays
+  const gf_ell* m = g->ell;
+  g->split = is_split_variant(iter_variant(group_variant(m), m->bslots, sizeof(double)));
+  if (g->split) {
+    std::vector<int32_t> sm(static_cast<size_t>(m->bslices + 2 * g->nmesh), 0);
+    for (int k = 0; k < g->nmesh; ++k)
+      std::fill(sm.begin() + bs[size_t(k)], sm.begin() + bs[size_t(k) + 1], k);
+    if (e == hipSuccess)
+      e = hipMalloc(&g->split_buf, size_t(m->n + m->bslices + 2 * g->nmesh) * sizeof(double));
+    if (e == hipSuccess) e = hipMalloc(&g->d_sl_ptr, bs.size() * 8);
+    if (e == hipSuccess) e = hipMalloc(&g->d_sl_mesh, sm.size() * 4);
+    if (e == hipSuccess) e = hipMemcpy(g->d_sl_ptr, bs.data(), bs.size() * 8, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(g->d_sl_mesh, sm.data(), sm.size() * 4, hipMemcpyHostToDevice);
+  }
   if (e == hipSuccess) e = hipMemcpy(g->d_sg_ptr, ptr.data(), ptr.size() * 8, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(g->d_sg_s0, s0.data(), s0.size() * 8, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(g->d_sg_s1, s1.data(), s1.size() * 8, hipMemcpyHostToDevice);
@@ -148,6 +171,13 @@ GroupBuffers buffers(gf_group* g) {
   G.sg_s0 = g->d_sg_s0;
   G.sg_s1 = g->d_sg_s1;
   G.part_sg = g->part_sg;
+  G.split = bsell && g->split;
+  G.z = g->split_buf;
+  G.part_sl = g->split_buf ? g->split_buf + m->n : nullptr;
+  G.rho2 = g->split_buf ? G.part_sl + m->bslices : nullptr;
+  G.sl_ptr = g->d_sl_ptr;
+  G.sl_mesh = g->d_sl_mesh;
+  G.it2 = g->d_sl_mesh ? g->d_sl_mesh + m->bslices : nullptr;
   G.rownnz = m->d_rownnz;
   G.diag = m->d_diag;
   G.dinv = m->d_dinv;
@@ -383,7 +413,9 @@ int gf_group_pcg(gf_ctx* ctx, gf_group* g, const double* b, double* x, const gf_
     hipGraph_t gr = nullptr;
     GF_HIP_CHECK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     hipError_t e = hipSuccess;
-    for (int it = 0; it < kChunk && e == hipSuccess; ++it) e = launch_group_iteration(ctx->stream, G);
+    for (int it = 0; it < kChunk && e == hipSuccess; ++it)
+      e = launch_group_iteration(ctx->stream, G, it & 1);
+    if (e == hipSuccess) e = launch_group_check(ctx->stream, G);
     hipError_t e2 = hipStreamEndCapture(ctx->stream, &gr);
     if (e == hipSuccess) e = e2;
     if (e == hipSuccess) e = hipGraphInstantiate(&g->graph, gr, nullptr, nullptr, 0);
@@ -406,7 +438,9 @@ int gf_group_pcg(gf_ctx* ctx, gf_group* g, const double* b, double* x, const gf_
       if (use_graph) {
         GF_HIP_CHECK(ctx, hipGraphLaunch(g->graph, ctx->stream));
       } else {
-        for (int it = 0; it < kChunk; ++it) GF_HIP_CHECK(ctx, launch_group_iteration(ctx->stream, G));
+        for (int it = 0; it < kChunk; ++it)
+          GF_HIP_CHECK(ctx, launch_group_iteration(ctx->stream, G, it & 1));
+        GF_HIP_CHECK(ctx, launch_group_check(ctx->stream, G));
       }
     }
     GF_HIP_CHECK(ctx, launch_group_x_finish(ctx->stream, G));

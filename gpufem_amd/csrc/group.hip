@@ -9,7 +9,9 @@
 // are skipped.  Workgroups take tiles in grid-stride order with the same
 // XCD remap as the single-system kernels.  One iteration is five launches:
 // SpMV + p.q partials, per-mesh alpha (a workgroup per mesh), update +
-// partials, per-mesh beta and stopping test (a workgroup per mesh), direction.
+// partials, per-mesh beta and stopping test (a workgroup per mesh), direction;
+// or two, for a matrix that stays in the last-level cache (k_gs_product,
+// k_gs_update).
 #include <cfloat>
 
 #include "device_common.hpp"
@@ -84,7 +86,13 @@ __global__ __launch_bounds__(kNT) void k_g_init(GroupBuffers G, int use_x0) {
       if (!use_x0) G.x[i] = 0.0;
       const double zi = G.dinv[i] * ri;
       G.r[i] = ri;
-      G.p[i] = zi;
+      if (G.split) {
+        const int64_t k = G.bsell_d == 2 ? lazy_index<2>(i, G.n) : lazy_index<3>(i, G.n);
+        G.z[k] = zi;
+        G.p[k] = 0.0;
+      } else {
+        G.p[i] = zi;
+      }
       rz = ri * zi;
       rr = ri * ri;
       bb = bi * bi;
@@ -118,6 +126,7 @@ __global__ __launch_bounds__(kNT) void k_g_init_finish(GroupBuffers G, double rt
     G.alpha[m] = 0.0;
     G.beta[m] = 0.0;
     G.it[m] = 0;
+    if (G.split) G.it2[m] = 0;
     G.status[m] = GF_OK;
     G.done[m] = (rr <= rtol2 * bb) || maxit <= 0;
     __threadfence();
@@ -294,6 +303,144 @@ __global__ __launch_bounds__(kNT) void k_g_beta(GroupBuffers G) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// The two-launch iteration of a group whose matrix stays in the last-level
+// cache (the single system's, solver.hip, with the scalars of each mesh).  A
+// workgroup belongs to one mesh, so it adds that mesh's partials itself: a few
+// hundred at most, one load per thread.  The two reduction launches and the
+// direction pass go (five launches before: 51.1 us an iteration on 64 Q4 plates
+// of 615 k rows in all, 33.4 now).
+// ---------------------------------------------------------------------------
+// whether mesh m runs iteration `it`; its lead thread records why not
+__device__ inline bool mesh_goes_on(const GroupBuffers& G, int m, int it, double rr, bool lead) {
+  if (!(rr <= G.st->rtol2 * G.bb[m]) && it < G.st->maxit) return true;
+  if (lead) {
+    G.rr[m] = rr;
+    G.it[m] = it;
+    G.done[m] = 1;
+  }
+  return false;
+}
+
+// One workgroup per slice.  done[m] changes inside a launch only when no
+// workgroup of the mesh writes a vector.
+template <int D>
+__global__ __launch_bounds__(64 * split_parts(D), D == 2 ? 6 : 4) void k_gs_product(
+    GroupBuffers G, int parity) {
+  __shared__ double sh[2 * (kNT / 64)];
+  const int64_t sl = logical_block();
+  if (sl >= G.bs.nslices) return;
+  const SplitSlice first = split_slice(sl, G.bs);
+  const int m = G.sl_mesh[sl];
+  const int done = G.st->done | G.done[m];
+  const int it = G.it2[parity * G.nmesh + m];
+  const double rz_old = G.rho2[(parity ^ 1) * G.nmesh + m];
+  const int64_t t0 = G.tile_ptr[m];
+  double rz, rr;
+  reduce_partials2(G.part + t0, G.part + G.ntiles + t0, int(G.tile_ptr[m + 1] - t0), &rz, &rr, sh);
+  const bool lead = threadIdx.x == 0 && sl == G.sl_ptr[m];
+  if (done || !mesh_goes_on(G, m, it, rr, lead)) return;
+  if (lead) G.rho2[parity * G.nmesh + m] = rz;
+  const LazyDirection<D> p{G.z, G.p, G.n / D, split_beta(it, rz, rz_old)};
+  double pq = 0.0;
+  for_rows_split<D>(first, int(G.bs.nslices), split_parts(D), G.bs, G.bval, G.bcol, p,
+                    [&](int32_t R, const double* acc) {
+#pragma unroll
+    for (int r = 0; r < D; ++r) {
+      G.q[int64_t(D) * R + r] = acc[r];
+      pq += p.at(R, r) * acc[r];
+    }
+  });
+  store_wave_sum(pq, G.part_sl + sl);
+}
+
+// One workgroup per tile of rows.
+template <int D>
+__global__ __launch_bounds__(kNT) void k_gs_update(GroupBuffers G, int parity) {
+  __shared__ double sh[2 * (kNT / 64)];
+  const int64_t t = logical_block();
+  if (t >= G.ntiles) return;
+  const int m = G.tile_mesh[t];
+  const int64_t i = G.tile_r0[t] + threadIdx.x, k = lazy_index<D>(i, G.n);
+  const bool row = i < G.tile_r1[t];
+  double x = 0.0, r = 0.0, q = 0.0, z = 0.0, po = 0.0, dinv = 0.0;
+  if (row) {
+    x = G.x[i];
+    r = G.r[i];
+    q = G.q[i];
+    dinv = G.dinv[i];
+    z = G.z[k];
+    po = G.p[k];
+  }
+  const int done = G.st->done | G.done[m];
+  const int it = G.it2[parity * G.nmesh + m];
+  const double rho = G.rho2[parity * G.nmesh + m];
+  const double beta = split_beta(it, rho, G.rho2[(parity ^ 1) * G.nmesh + m]);
+  const int64_t s0 = G.sl_ptr[m];
+  const double pq = reduce_partials(G.part_sl + s0, int(G.sl_ptr[m + 1] - s0), sh);
+  if (done) return;
+  const bool lead = threadIdx.x == 0 && t == G.tile_ptr[m];
+  if (!(pq > 0.0)) {
+    if (lead) {
+      G.it[m] = it;
+      G.status[m] = GF_ERR_BREAKDOWN;
+      G.done[m] = 1;
+    }
+    return;
+  }
+  const double alpha = rho / pq;
+  double rz = 0.0, rr = 0.0;
+  if (row) {
+    const double pi = z + beta * po;
+    const double ri = r - alpha * q;
+    const double zi = dinv * ri;
+    G.x[i] = x + alpha * pi;
+    G.r[i] = ri;
+    G.z[k] = zi;
+    G.p[k] = pi;
+    rz = ri * zi;
+    rr = ri * ri;
+  }
+  block_sum2(&rz, &rr, sh);
+  if (threadIdx.x == 0) {
+    G.part[t] = rz;
+    G.part[G.ntiles + t] = rr;
+  }
+  if (lead) G.it2[(parity ^ 1) * G.nmesh + m] = it + 1;
+}
+
+// The stopping tests the next iteration (of parity 0) would make, one
+// workgroup per mesh; the last to finish (an arrival counter) sets the done
+// flag when every mesh is done.
+__global__ __launch_bounds__(kNT) void k_gs_check(GroupBuffers G) {
+  GroupState* st = G.st;
+  if (st->done) return;
+  __shared__ double sh[2 * (kNT / 64)];
+  const int m = blockIdx.x;
+  if (!G.done[m]) {
+    const int64_t t0 = G.tile_ptr[m];
+    double rz, rr;
+    reduce_partials2(G.part + t0, G.part + G.ntiles + t0, int(G.tile_ptr[m + 1] - t0), &rz, &rr,
+                     sh);
+    if (threadIdx.x == 0) {
+      G.rr[m] = rr;
+      G.it[m] = G.it2[m];
+      (void)mesh_goes_on(G, m, G.it2[m], rr, true);
+    }
+  }
+  if (threadIdx.x == 0) {
+    __threadfence();
+    if (atomicAdd(&st->arrived, 1) == G.nmesh - 1) {
+      __threadfence();
+      int all = 1;
+      for (int j = 0; j < G.nmesh; ++j)
+        all &= __hip_atomic_load(&G.done[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      st->arrived = 0;
+      if (all) st->done = 1;
+    }
+  }
+}
+
 // x += alpha p with this iteration's p (alpha = 0 for meshes done before
 // it), then p = D^-1 r + beta p.  The iteration that finishes the group
 // returns here before the x update (done is set); k_g_x_finish applies it.
@@ -391,9 +538,21 @@ hipError_t launch_group_setup(hipStream_t s, const GroupBuffers& G, int use_x0, 
   return hipGetLastError();
 }
 
-hipError_t launch_group_iteration(hipStream_t s, const GroupBuffers& G) {
+hipError_t launch_group_iteration(hipStream_t s, const GroupBuffers& G, int parity) {
   hipError_t e;
   const dim3 g(G.nblocks), t(kNT);
+  if (G.split) {
+    // one workgroup per slice / per tile, in multiples of 8 for the XCD remap
+    const dim3 gp(unsigned((G.bs.nslices + 7) & ~int64_t(7)));
+    const dim3 gu(unsigned((G.ntiles + 7) & ~int64_t(7)));
+    const int d = G.bsell_d;
+    if (d == 2) hipLaunchKernelGGL(k_gs_product<2>, gp, dim3(64 * split_parts(2)), 0, s, G, parity);
+    else hipLaunchKernelGGL(k_gs_product<3>, gp, dim3(64 * split_parts(3)), 0, s, G, parity);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if (d == 2) hipLaunchKernelGGL(k_gs_update<2>, gu, t, 0, s, G, parity);
+    else hipLaunchKernelGGL(k_gs_update<3>, gu, t, 0, s, G, parity);
+    return hipGetLastError();
+  }
   const dim3 gs(G.nsg < 65536 ? (G.nsg > 0 ? G.nsg : 1) : 65536);
   if (G.bsell_d == 2) hipLaunchKernelGGL(k_g_spmv_pq_bs<2>, gs, t, 0, s, G);
   else if (G.bsell_d == 3) hipLaunchKernelGGL(k_g_spmv_pq_bs<3>, gs, t, 0, s, G);
@@ -415,7 +574,14 @@ hipError_t launch_group_iteration(hipStream_t s, const GroupBuffers& G) {
   return hipGetLastError();
 }
 
+hipError_t launch_group_check(hipStream_t s, const GroupBuffers& G) {
+  if (!G.split) return hipSuccess;  // k_g_beta tests
+  hipLaunchKernelGGL(k_gs_check, dim3(G.nmesh), dim3(kNT), 0, s, G);
+  return hipGetLastError();
+}
+
 hipError_t launch_group_x_finish(hipStream_t s, const GroupBuffers& G) {
+  if (G.split) return hipSuccess;  // x follows every iteration
   hipLaunchKernelGGL(k_g_x_finish, dim3(G.nblocks), dim3(kNT), 0, s, G);
   return hipGetLastError();
 }

@@ -45,6 +45,15 @@ struct GroupBuffers {
   const int64_t* sg_s0;    // [nsg] first slice
   const int64_t* sg_s1;    // [nsg] end slice
   double* part_sg;         // [nsg] p.q partials
+  // two-launch iteration (split): z and p component-major, one partial p.q per
+  // slice, rho and the iteration count of each mesh by parity
+  bool split;
+  double* z;
+  const int64_t* sl_ptr;   // [nmesh+1] first slice of each mesh
+  const int32_t* sl_mesh;  // [nslices]
+  double* part_sl;         // [nslices]
+  double* rho2;            // [2][nmesh]
+  int32_t* it2;            // [2][nmesh]
   double *rho, *alpha, *beta, *rr, *bb, *pen;  // [nmesh]
   int32_t *it, *done, *status;                 // [nmesh]
   GroupState* st;
@@ -57,7 +66,10 @@ hipError_t launch_group_penalty(hipStream_t s, const GroupBuffers& G, double coe
                                 int64_t nd);
 hipError_t launch_group_setup(hipStream_t s, const GroupBuffers& G, int use_x0, double rtol,
                               int maxit);
-hipError_t launch_group_iteration(hipStream_t s, const GroupBuffers& G);
+hipError_t launch_group_iteration(hipStream_t s, const GroupBuffers& G, int parity);
+// after an even number of iterations: the stopping tests of the residuals they
+// left (the two-launch iteration only)
+hipError_t launch_group_check(hipStream_t s, const GroupBuffers& G);
 // x += alpha p of the group's last iteration (once, after the loop)
 hipError_t launch_group_x_finish(hipStream_t s, const GroupBuffers& G);
 hipError_t launch_group_residual(hipStream_t s, const GroupBuffers& G, double* out);

@@ -246,13 +246,6 @@ __device__ inline double phase_split(const PcgBuffers& B, SplitSlice first, int 
   return pq;
 }
 
-// the sum over wave 0's lanes, written by lane 0
-__device__ inline void store_wave_sum(double v, double* out) {
-  if (threadIdx.x >= 64) return;
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  if (threadIdx.x == 0) *out = v;
-}
-
 // kRows rows of a thread at a time: the loads of the first ones are issued
 // before the scalars of the iteration are known (their latency and the
 // reduction's overlap).  Row i = D node + e of the solver's vectors is entry
@@ -262,17 +255,12 @@ struct SplitRows {
   double x[kRows], z[kRows], p[kRows], r[kRows], q[kRows], d[kRows];
 };
 template <int D>
-__device__ inline int64_t lazy_index(const PcgBuffers& B, int64_t i) {
-  const uint32_t node = uint32_t(i) / D, e = uint32_t(i) - node * D;
-  return int64_t(e) * (B.n / D) + node;
-}
-template <int D>
 __device__ inline void split_load(const PcgBuffers& B, int64_t base, int64_t stride, SplitRows* v) {
 #pragma unroll
   for (int u = 0; u < kRows; ++u) {
     const int64_t i = base + u * stride;
     if (i < B.n) {
-      const int64_t k = lazy_index<D>(B, i);
+      const int64_t k = lazy_index<D>(i, B.n);
       v->z[u] = B.z[k];
       v->p[u] = B.p[k];
       v->x[u] = B.x[i];
@@ -294,7 +282,7 @@ __device__ inline void phase_split_update(const PcgBuffers& B, int lb, int slot,
     for (int u = 0; u < kRows; ++u) {
       const int64_t i = base + u * stride;
       if (i < B.n) {
-        const int64_t k = lazy_index<D>(B, i);
+        const int64_t k = lazy_index<D>(i, B.n);
         const double pi = v.z[u] + beta * v.p[u];
         const double ri = v.r[u] - alpha * v.q[u];
         const double zi = B.dinv ? v.d[u] * ri : ri;
@@ -335,10 +323,6 @@ __device__ inline void split_breakdown(const PcgBuffers& B, int it, bool lead) {
   B.st->status = GF_ERR_BREAKDOWN;
   B.st->done = 1;
 }
-__device__ inline double split_beta(int it, double rz, double rz_old) {
-  return it > 0 ? rz / rz_old : 0.0;
-}
-
 // First launch: the stopping test, beta and q = K p.  `done` changes inside a
 // launch only when none of its workgroups writes a vector, so one that starts
 // late and reads it set leaves nothing undone.
@@ -411,7 +395,7 @@ __global__ __launch_bounds__(kNT) void k_pcg_init(PcgBuffers B, int use_x0) {
     const double zi = B.dinv ? B.dinv[i] * ri : ri;
     B.r[i] = ri;
     if constexpr (SOA > 1) {
-      const int64_t k = lazy_index<SOA>(B, i);
+      const int64_t k = lazy_index<SOA>(i, B.n);
       B.z[k] = zi;
       B.p[k] = 0.0;
     } else {

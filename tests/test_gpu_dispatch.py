@@ -88,3 +88,25 @@ def test_two_launch_iteration_breakdown(gpu_ctx):
         assert s.code == gf.GF_ERR_BREAKDOWN and s.iterations == 0
         x, s = gpu_ctx.pcg(K, 0.0 * f, schedule=sched)
         assert s.converged and s.iterations == 0 and not x.any()
+
+
+def test_group_two_launch_iteration(gpu_ctx):
+    """A grouped solve whose matrix stays in the last-level cache, meshes of one
+    element to several slices: each mesh as solved alone (its own stopping
+    test), the schedules bitwise alike, a capped solve stopping at the cap."""
+    for t, sizes in ((gf.GF_Q4, [(1, 1), (40, 20), (7, 7), (64, 1)]),
+                     (gf.GF_BRICK8, [(3, 2, 2), (1, 1, 1), (9, 8, 7)])):
+        probs = [P.structured(t, *s) for s in sizes]
+        G = gpu_ctx.group(probs)
+        G.assemble()
+        G.apply_penalty()
+        x, st, its = G.pcg(rtol=1e-10)
+        xk, sk, ik = G.pcg(rtol=1e-10, schedule=gf.GF_SCHED_KERNELS)
+        assert np.array_equal(x, xk) and np.array_equal(its, ik)
+        for p, xs, it in zip(probs, G.split(x), its):
+            q, K = assembled(gpu_ctx, t, *(list(sizes[probs.index(p)]) + [0])[:3])
+            xo, so = gpu_ctx.pcg(K, q.f, rtol=1e-10)
+            assert abs(int(it) - so.iterations) <= 2 + so.iterations // 100
+            assert np.linalg.norm(xs - xo) <= 1e-9 * np.linalg.norm(xo)
+        xc, sc, ic = G.pcg(rtol=1e-10, maxit=5, verify=0, raise_on_fail=False)
+        assert sc.code == gf.GF_ERR_NOCONV and ic.max() == 5
