@@ -32,6 +32,7 @@ constexpr int kCin = 16;     // input channels (features, zero-padded)
 constexpr int kCout = 16;    // output channels (first kOutUsed are used)
 constexpr int kOutUsed = 3;
 constexpr float kSlope = 0.1f;
+constexpr int64_t kSmallParts = 256 * 256;  // bias and loss partials
 
 enum Buf {
   B_IN = 0, B_A0, B_CAT0, B_A1, B_CAT1, B_A2, B_CAT2, B_A3, B_B2, B_C2, B_B1, B_C1, B_B0, B_C0,
@@ -256,18 +257,19 @@ hipError_t backward(hipStream_t s, gf_nn* net, const uint16_t* input, int batch)
     w.dz_ld = l.out.ld;
     w.dz_off = l.out.off;
     w.part = net->wpart;
+    w.bpart = net->spart;
     w.batch = batch;
     w.vin = net->lv[l.in.level];
     w.vout = net->lv[l.out.level];
     w.cin = l.cin;
     w.cout = l.cout;
     w.stride = l.stride;
-    w.nchunk = wgrad_chunks(nvo);
+    w.nchunk = wgrad_chunks(nvo, l.cin, l.cout);
     w.chunk = ((nvo + w.nchunk - 1) / w.nchunk + 63) / 64 * 64;
-    if (int64_t(w.nchunk) * 27 * l.cin * l.cout > net->wpart_len) return hipErrorInvalidValue;
-    e = launch_wgrad(s, w, net->g + l.w_off);
-    if (e != hipSuccess) return e;
-    e = launch_bias_grad(s, dz, l.out.ld, l.out.off, nvo, l.cout, net->spart, net->g + l.b_off);
+    if (int64_t(w.nchunk) * 27 * l.cin * l.cout > net->wpart_len ||
+        int64_t(w.nchunk) * l.cout > kSmallParts)
+      return hipErrorInvalidValue;
+    e = launch_wgrad(s, w, net->g + l.w_off, net->g + l.b_off);
     if (e != hipSuccess) return e;
     if (!l.need_dx) continue;
     ConvArgs a{};
@@ -332,14 +334,16 @@ int gf_nn_create(gf_ctx* ctx, int32_t nx, int32_t ny, int32_t nz, int32_t batch_
     e = dalloc(net, &net->pred, size_t(voxels(net, 0, batch_max)) * kCout * sizeof(float));
   int64_t wl = 0;
   for (const Layer& l : net->layers)
-    wl = std::max<int64_t>(wl, int64_t(wgrad_chunks(voxels(net, l.out.level, batch_max))) * 27 *
-                                   l.cin * l.cout);
+    // (a smaller batch never takes more chunks)
+    wl = std::max<int64_t>(
+        wl, int64_t(wgrad_chunks(voxels(net, l.out.level, batch_max), l.cin, l.cout)) * 27 *
+                l.cin * l.cout);
   net->wpart_len = wl;
   if (e == hipSuccess) e = dalloc(net, &net->wpart, size_t(wl) * sizeof(float));
-  if (e == hipSuccess) e = dalloc(net, &net->spart, size_t(256 * 256) * sizeof(float));
+  if (e == hipSuccess) e = dalloc(net, &net->spart, size_t(kSmallParts) * sizeof(float));
   if (e == hipSuccess) e = dalloc(net, &net->loss, sizeof(float));
   for (Layer& l : net->layers) {
-    const size_t fb = size_t(27) * l.cin * l.cout * sizeof(uint16_t);
+    const size_t fb = conv_fragments(l.cin, l.cout) * sizeof(uint16_t);
     if (e == hipSuccess) e = dalloc(net, &l.wf, fb);
     if (e == hipSuccess && l.need_dx) e = dalloc(net, &l.wt, fb);
   }
@@ -515,7 +519,7 @@ int gf_nn_conv3d(gf_ctx* ctx, const uint16_t* in_dev, int32_t batch, const int32
   GF_HIP_CHECK(ctx, hipSetDevice(ctx->device));
   // fragments of the weights W[27][cin][cout] (or, transposed, W[27][cout][cin])
   uint16_t* wf = nullptr;
-  GF_HIP_CHECK(ctx, hipMalloc(&wf, size_t(27) * cin * cout * sizeof(uint16_t)));
+  GF_HIP_CHECK(ctx, hipMalloc(&wf, conv_fragments(cin, cout) * sizeof(uint16_t)));
   hipError_t e = transposed ? launch_arrange(ctx->stream, w_dev, wf, cout, cin, 1)
                             : launch_arrange(ctx->stream, w_dev, wf, cin, cout, 0);
   ConvArgs a{};
@@ -568,15 +572,13 @@ int gf_nn_conv3d_wgrad(gf_ctx* ctx, const uint16_t* x_dev, int32_t batch, const 
   w.cout = cout;
   w.stride = stride;
   const int64_t nvo = int64_t(batch) * w.vout.nodes();
-  w.nchunk = wgrad_chunks(nvo);
+  w.nchunk = wgrad_chunks(nvo, cin, cout);
   w.chunk = ((nvo + w.nchunk - 1) / w.nchunk + 63) / 64 * 64;
   float* part = nullptr;
-  GF_HIP_CHECK(ctx, hipMalloc(&part, (size_t(w.nchunk) * 27 * cin * cout + 256 * 256) * sizeof(float)));
+  GF_HIP_CHECK(ctx, hipMalloc(&part, size_t(w.nchunk) * (27 * size_t(cin) + 1) * cout * sizeof(float)));
   w.part = part;
-  hipError_t e = launch_wgrad(ctx->stream, w, dw_dev);
-  if (e == hipSuccess && db_dev)
-    e = launch_bias_grad(ctx->stream, dz_dev, cout, 0, nvo, cout,
-                         part + size_t(w.nchunk) * 27 * cin * cout, db_dev);
+  w.bpart = db_dev ? part + size_t(w.nchunk) * 27 * cin * cout : nullptr;
+  hipError_t e = launch_wgrad(ctx->stream, w, dw_dev, db_dev);
   hipError_t e2 = hipStreamSynchronize(ctx->stream);
   (void)hipFree(part);
   if (e == hipSuccess) e = e2;

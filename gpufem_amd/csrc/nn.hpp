@@ -47,7 +47,8 @@ struct WgradArgs {
   int x_ld, x_off;
   const uint16_t* dz;
   int dz_ld, dz_off;
-  float* part;  // [nchunk][27][cin][cout]
+  float* part;   // [nchunk][27][cin][cout]
+  float* bpart;  // [nchunk][cout] sums of dz (null: none)
   int batch;
   Vol vin, vout;
   int cin, cout, stride;
@@ -56,8 +57,11 @@ struct WgradArgs {
 };
 
 hipError_t launch_conv(hipStream_t s, const ConvArgs& a);
-int wgrad_chunks(int64_t voxels);
-hipError_t launch_wgrad(hipStream_t s, const WgradArgs& a, float* dw);
+int wgrad_chunks(int64_t voxels, int cin, int cout);
+// dw, and db[c] = sum over voxels of dz[v][c] (null: none)
+hipError_t launch_wgrad(hipStream_t s, const WgradArgs& a, float* dw, float* db);
+// elements a fragment buffer of launch_arrange holds
+size_t conv_fragments(int cin, int cout);
 // fp32 master weights W[27][cin][cout] -> MFMA fragments; transposed
 // swaps the roles of input and output channels (for the data gradient)
 hipError_t launch_arrange(hipStream_t s, const float* w, uint16_t* wf, int cin, int cout,
@@ -65,9 +69,6 @@ hipError_t launch_arrange(hipStream_t s, const float* w, uint16_t* wf, int cin, 
 // y > 0 ? dy : slope * dy, in place on the channel slice [off, off + c)
 hipError_t launch_act_bwd(hipStream_t s, uint16_t* dy, int dy_ld, int dy_off, const uint16_t* y,
                           int y_ld, int y_off, int64_t voxels, int c, float slope);
-// db[c] = sum over voxels of dz[v][c]
-hipError_t launch_bias_grad(hipStream_t s, const uint16_t* dz, int ld, int off, int64_t voxels,
-                            int c, float* part, float* db);
 // vertex-centred trilinear prolongation coarse (vc) -> fine (vf = 2 vc - 1)
 // and its adjoint; both overwrite their output slice
 hipError_t launch_prolong(hipStream_t s, const uint16_t* in, int in_ld, int in_off, Vol vc,

@@ -93,7 +93,9 @@ def test_two_launch_iteration_breakdown(gpu_ctx):
 def test_group_two_launch_iteration(gpu_ctx):
     """A grouped solve whose matrix stays in the last-level cache, meshes of one
     element to several slices: each mesh as solved alone (its own stopping
-    test), the schedules bitwise alike, a capped solve stopping at the cap."""
+    test) as nearly as the single system's own variants agree (the slender plate
+    cannot reach this tolerance in FP64: they take 1733 to 2002 iterations), the
+    schedules bitwise alike, a capped solve stopping at the cap."""
     for t, sizes in ((gf.GF_Q4, [(1, 1), (40, 20), (7, 7), (64, 1)]),
                      (gf.GF_BRICK8, [(3, 2, 2), (1, 1, 1), (9, 8, 7)])):
         probs = [P.structured(t, *s) for s in sizes]
@@ -105,8 +107,13 @@ def test_group_two_launch_iteration(gpu_ctx):
         assert np.array_equal(x, xk) and np.array_equal(its, ik)
         for p, xs, it in zip(probs, G.split(x), its):
             q, K = assembled(gpu_ctx, t, *(list(sizes[probs.index(p)]) + [0])[:3])
-            xo, so = gpu_ctx.pcg(K, q.f, rtol=1e-10)
-            assert abs(int(it) - so.iterations) <= 2 + so.iterations // 100
-            assert np.linalg.norm(xs - xo) <= 1e-9 * np.linalg.norm(xo)
+            alone = []
+            for v in (0, 3, 4, 9 if t == gf.GF_Q4 else 10):
+                gpu_ctx.tune(K, v)
+                alone.append(gpu_ctx.pcg(K, q.f, rtol=1e-10))
+            xo, counts = alone[0][0], [s.iterations for _, s in alone]
+            apart = max(np.linalg.norm(xv - xo) for xv, _ in alone)
+            assert abs(int(it) - counts[0]) <= 2 + counts[0] // 100 + max(counts) - min(counts)
+            assert np.linalg.norm(xs - xo) <= 1e-9 * np.linalg.norm(xo) + 2 * apart
         xc, sc, ic = G.pcg(rtol=1e-10, maxit=5, verify=0, raise_on_fail=False)
         assert sc.code == gf.GF_ERR_NOCONV and ic.max() == 5
