@@ -102,25 +102,22 @@ __global__ __launch_bounds__(kNT) void k_b_init_finish(MultiBuffers B, int nb, i
 // q = K p and the per-column partials of p.q.  Launched at three workgroups
 // per CU (padded LDS), i.e. three waves per SIMD, so the compiler may spend up
 // to 168 registers keeping every load of a step in flight.
-template <int S, int D, int NB = 2>
+template <int S, int D, int PARTS, int NB = 2>
 __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_b_spmm_pq_bs(
     MultiBuffers B) {
   const MultiState<S>* st = static_cast<const MultiState<S>*>(B.st);
   if (st->done) return;
-  __shared__ double sh[kNT * kCB];
+  __shared__ double sh[spmm_lds_values<D, kCB, PARTS>()];
   double pq[kCB] = {};
   constexpr bool share = Chunks<S, kCB>::L >= NB * (D * D / 2);
-  for_chunk_node_rows<S, D, double, double, false, NB, true, kCB, share>(
-      spmm_args(B), B.val, B.p, [&](int32_t R, int c0, const double (*acc)[kCB]) {
+  for_chunk_node_rows<S, D, double, double, false, NB, true, kCB, share, PARTS>(
+      spmm_args(B), B.val, B.p, sh, [&](int32_t R, int r, int c0, const double* acc) {
+        const int64_t o = (int64_t(D) * R + r) * S;
+        double pv[kCB];
+        load_split<S, kCB>(B.p + o, c0, pv);
+        store_split<S, kCB>(B.q + o, c0, acc);
 #pragma unroll
-        for (int r = 0; r < D; ++r) {
-          const int64_t o = (int64_t(D) * R + r) * S;
-          double pv[kCB];
-          load_split<S, kCB>(B.p + o, c0, pv);
-          store_split<S, kCB>(B.q + o, c0, acc[r]);
-#pragma unroll
-          for (int j = 0; j < kCB; ++j) pq[j] += pv[j] * acc[r][j];
-        }
+        for (int j = 0; j < kCB; ++j) pq[j] += pv[j] * acc[j];
       });
   chunk_partials<S, true, kCB>(pq, sh, B.part1);
 }
@@ -129,10 +126,9 @@ template <int S, int D>
 __global__ __launch_bounds__(kNT) void k_b_spmm_bs(MultiBuffers B, const double* __restrict__ xin,
                                                    double* __restrict__ yout) {
   for_chunk_node_rows<S, D, double, double, false, 2, true, kCB>(
-      spmm_args(B), B.val, xin, [&](int32_t R, int c0, const double (*acc)[kCB]) {
-#pragma unroll
-        for (int r = 0; r < D; ++r)
-          store_split<S, kCB>(yout + (int64_t(D) * R + r) * S, c0, acc[r]);
+      spmm_args(B), B.val, xin, static_cast<double*>(nullptr),
+      [&](int32_t R, int r, int c0, const double* acc) {
+        store_split<S, kCB>(yout + (int64_t(D) * R + r) * S, c0, acc);
       });
 }
 
@@ -358,9 +354,14 @@ hipError_t launch_spmm_pq(hipStream_t s, const MultiBuffers& B) {
   const dim3 g(B.nblocks), t(kNT);
   // padded LDS: three workgroups per CU (four fit) keep each XCD's rows in
   // flight (and the 32-wide rows of p they gather) closer to what its L2 holds
-  if (B.bsell_d == 2) hipLaunchKernelGGL((k_b_spmm_pq_bs<S, 2>), g, t, B.spmm_lds, s, B);
-  else if (B.bsell_d == 3) hipLaunchKernelGGL((k_b_spmm_pq_bs<S, 3>), g, t, B.spmm_lds, s, B);
-  else hipLaunchKernelGGL(k_b_spmm_pq<S>, g, t, 0, s, B);
+  if (B.bsell_d == 2)
+    hipLaunchKernelGGL((k_b_spmm_pq_bs<S, 2, 1>), g, t, B.spmm_lds, s, B);
+  else if (B.bsell_d == 3 && spmm_parts<S>(B.bs.nslices) > 1)
+    hipLaunchKernelGGL((k_b_spmm_pq_bs<S, 3, 4>), g, t, 0, s, B);
+  else if (B.bsell_d == 3)
+    hipLaunchKernelGGL((k_b_spmm_pq_bs<S, 3, 1>), g, t, B.spmm_lds, s, B);
+  else
+    hipLaunchKernelGGL(k_b_spmm_pq<S>, g, t, 0, s, B);
   return hipGetLastError();
 }
 

@@ -251,7 +251,13 @@ __device__ inline void ell_row_chunk(const SpmmArgs& A, const VT* __restrict__ v
 }
 
 // Block-sliced copy: positions of the node-row permutation in grid-stride
-// order, G per workgroup pass; f(R, c0, acc) gets the D rows of node row R.
+// order, G per workgroup pass; f(R, r, c0, acc) gets row r of node row R, for
+// each r.
+// PARTS = 4: the four waves share the rows of a pass (a quarter as many), each
+// takes a quarter of a row's blocks, and wave r adds the four partial rows r (in
+// wave order; shp: PARTS * 64 * D * KC values of LDS).  For 3D matrices of fewer
+// passes than workgroups fit the chip (spmm_parts), whose single pass is one
+// serial chain of up to 81 blocks.
 // DIFF: the values are the difference form of the FP32 copy (see bsell_row):
 // off-diagonal blocks multiply x_J - x_R, the diagonal slot (node column R)
 // holds the block row sum and multiplies x_R.
@@ -262,20 +268,27 @@ __device__ inline void ell_row_chunk(const SpmmArgs& A, const VT* __restrict__ v
 // them (a cross-lane permute through the LDS crossbar) instead of each loading
 // all of them; the vector-memory path then carries mostly the gathers of x.
 template <int S, int D, class T, class VT, bool DIFF = false, int NB = 2, bool SPLIT = false,
-          int KC = kC, bool SHARE = false, class F>
+          int KC = kC, bool SHARE = false, int PARTS = 1, class F>
 __device__ inline void for_chunk_node_rows(const SpmmArgs& A, const VT* __restrict__ val,
-                                           const T* __restrict__ xin, F&& f) {
+                                           const T* __restrict__ xin, T* shp, F&& f) {
   static_assert(!(DIFF && SPLIT), "the difference form reads x_R in the contiguous order");
+  static_assert(PARTS == 1 || PARTS == kNT / 64, "a wave per part");
   int g, c0;
   chunk_lane<S, KC>(&g, &c0);
+  constexpr int G = Chunks<S, KC>::G / PARTS;  // rows per pass
+  // a pass is whole or not at all where its waves meet at barriers
+  static_assert(PARTS == 1 || 64 % G == 0, "a pass inside a slice");
+  g %= G;
+  const int part = PARTS == 1 ? 0 : int(threadIdx.x) >> 6;
   const int64_t npos = A.bs.nslices * 64;
-  const int64_t stride = int64_t(gridDim.x) * Chunks<S, KC>::G;
-  for (int64_t pos = int64_t(logical_block()) * Chunks<S, KC>::G + g; pos < npos; pos += stride) {
+  const int64_t stride = int64_t(gridDim.x) * G;
+  for (int64_t pos = int64_t(logical_block()) * G + g; pos < npos; pos += stride) {
     const int32_t R = A.bs.perm[pos];
-    if (R < 0) continue;
+    if (PARTS == 1 && R < 0) continue;
     const int lp = int(pos & 63);
-    const int32_t cnt = A.rownnz[int64_t(D) * R] / D;
-    const int64_t b0 = A.bs.sptr[pos >> 6];
+    const int32_t all = R >= 0 ? A.rownnz[int64_t(D) * R] / D : 0;
+    const int32_t from = all * part / PARTS, cnt = all * (part + 1) / PARTS - from;
+    const int64_t b0 = A.bs.sptr[pos >> 6] + from;
     T acc[D][KC];
 #pragma unroll
     for (int r = 0; r < D; ++r)
@@ -287,8 +300,9 @@ __device__ inline void for_chunk_node_rows(const SpmmArgs& A, const VT* __restri
     };
     T xr[D][KC];
     if constexpr (DIFF) {
+      const int64_t row = int64_t(D) * (R >= 0 ? R : 0);
 #pragma unroll
-      for (int e = 0; e < D; ++e) load_chunk(xin + (int64_t(D) * R + e) * S + c0, xr[e]);
+      for (int e = 0; e < D; ++e) load_chunk(xin + (row + e) * S + c0, xr[e]);
     }
     // x_J - x_R off the diagonal (DIFF)
     auto rel = [&](int64_t c, T (*xv)[KC]) {
@@ -393,8 +407,48 @@ __device__ inline void for_chunk_node_rows(const SpmmArgs& A, const VT* __restri
             for (int j = 0; j < KC; ++j) acc[r][j] += v[r * D + e] * xv[e][j];
       }
     }
-    f(R, c0, acc);
+    if constexpr (PARTS == 1) {
+#pragma unroll
+      for (int r = 0; r < D; ++r) f(R, r, c0, acc[r]);
+    } else {
+      const int lane = threadIdx.x & 63;
+      T* mine = shp + (part * D * KC) * 64 + lane;
+#pragma unroll
+      for (int r = 0; r < D; ++r)
+#pragma unroll
+        for (int j = 0; j < KC; ++j) mine[(r * KC + j) * 64] = acc[r][j];
+      __syncthreads();
+      if (part < D && R >= 0) {
+        T t[KC];
+#pragma unroll
+        for (int j = 0; j < KC; ++j) {
+          t[j] = shp[(part * KC + j) * 64 + lane];
+#pragma unroll
+          for (int w = 1; w < PARTS; ++w) t[j] += shp[((w * D + part) * KC + j) * 64 + lane];
+        }
+        f(R, part, c0, t);
+      }
+      __syncthreads();  // the next pass writes the partial rows
+    }
   }
+}
+
+// Shares of a 3D row's blocks: four below as many passes as workgroups are
+// co-resident (three per CU of 256).  Iterations measured, four shares against
+// one: Brick20 20x17x13, 12 load cases (317 passes) 77.5 / 101.7 us in FP64, 68.2
+// / 76.4 mixed; Brick20 8^3, 32 (84) 59.5 / 67.3 and 65.9 / 72.2; Brick20 24^3,
+// 32 (1896) 334 / 326 and 173 / 172; Brick8 40^3, 24 (2154) 250 / 249 and 148 /
+// 141.  2D rows (at most 21 blocks) only lose: Q8 100x60 38.4 / 35.8.
+template <int S>
+inline int spmm_parts(int64_t nslices) {
+  return nslices * 64 / Chunks<S>::G < 768 ? kNT / 64 : 1;
+}
+
+// LDS values of a kernel that forms partial rows (PARTS > 1) and then column
+// partials in it
+template <int D, int KC, int PARTS>
+constexpr int spmm_lds_values() {
+  return PARTS > 1 && PARTS * 64 * D * KC > kNT * KC ? PARTS * 64 * D * KC : kNT * KC;
 }
 
 // per-column workgroup sums of the lanes' chunk partials into part[k][block]

@@ -92,10 +92,9 @@ __global__ __launch_bounds__(kNT) void k_mm_refresh(MixedMultiBuffers B, int set
       row(i, c0, kx);
     });
   } else {
-    for_chunk_node_rows<S, D>(spmm_args(B), B.val, B.x,
-                              [&](int32_t R, int c0, const double (*acc)[kC]) {
-#pragma unroll
-                                for (int r = 0; r < D; ++r) row(int64_t(D) * R + r, c0, acc[r]);
+    for_chunk_node_rows<S, D>(spmm_args(B), B.val, B.x, static_cast<double*>(nullptr),
+                              [&](int32_t R, int r, int c0, const double* acc) {
+                                row(int64_t(D) * R + r, c0, acc);
                               });
   }
   double* out = setup ? B.part2 : B.part3;
@@ -150,11 +149,11 @@ __global__ __launch_bounds__(kNT) void k_mm_setup_finish(MixedMultiBuffers B, in
   }
 }
 
-template <int S, int D>
+template <int S, int D, int PARTS>
 __global__ __launch_bounds__(kNT) void k_mm_spmm_pq(MixedMultiBuffers B) {
   const MMState<S>* st = static_cast<const MMState<S>*>(B.st);
   if (st->done) return;
-  __shared__ double sh[kNT * kC];
+  __shared__ double sh[spmm_lds_values<D, kC, PARTS>()];
   double pq[kC] = {};
   auto row = [&](int64_t i, int c0, const float* acc) {
     const int64_t o = i * S + c0;
@@ -172,11 +171,9 @@ __global__ __launch_bounds__(kNT) void k_mm_spmm_pq(MixedMultiBuffers B) {
     });
   } else {
     constexpr bool share = Chunks<S>::L >= 2 * (D * D / 4);
-    for_chunk_node_rows<S, D, float, float, true, 2, false, kC, share>(
-        spmm_args(B), B.val32, B.p, [&](int32_t R, int c0, const float (*acc)[kC]) {
-#pragma unroll
-          for (int r = 0; r < D; ++r) row(int64_t(D) * R + r, c0, acc[r]);
-        });
+    for_chunk_node_rows<S, D, float, float, true, 2, false, kC, share, PARTS>(
+        spmm_args(B), B.val32, B.p, reinterpret_cast<float*>(sh),
+        [&](int32_t R, int r, int c0, const float* acc) { row(int64_t(D) * R + r, c0, acc); });
   }
   chunk_partials<S>(pq, sh, B.part1);
 }
@@ -365,9 +362,14 @@ template <int S>
 hipError_t iteration_s(hipStream_t s, const MixedMultiBuffers& B) {
   hipError_t e;
   const dim3 g(B.nblocks), t(kNT);
-  if (B.bsell_d == 2) hipLaunchKernelGGL((k_mm_spmm_pq<S, 2>), g, t, 0, s, B);
-  else if (B.bsell_d == 3) hipLaunchKernelGGL((k_mm_spmm_pq<S, 3>), g, t, 0, s, B);
-  else hipLaunchKernelGGL((k_mm_spmm_pq<S, 0>), g, t, 0, s, B);
+  if (B.bsell_d == 2)
+    hipLaunchKernelGGL((k_mm_spmm_pq<S, 2, 1>), g, t, 0, s, B);
+  else if (B.bsell_d == 3 && spmm_parts<S>(B.bs.nslices) > 1)
+    hipLaunchKernelGGL((k_mm_spmm_pq<S, 3, 4>), g, t, 0, s, B);
+  else if (B.bsell_d == 3)
+    hipLaunchKernelGGL((k_mm_spmm_pq<S, 3, 1>), g, t, 0, s, B);
+  else
+    hipLaunchKernelGGL((k_mm_spmm_pq<S, 0, 1>), g, t, 0, s, B);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   hipLaunchKernelGGL(k_mm_alpha<S>, dim3(S), t, 0, s, B, B.nblocks);
   if ((e = hipGetLastError()) != hipSuccess) return e;

@@ -117,3 +117,25 @@ def test_group_two_launch_iteration(gpu_ctx):
             assert np.linalg.norm(xs - xo) <= 1e-9 * np.linalg.norm(xo) + 2 * apart
         xc, sc, ic = G.pcg(rtol=1e-10, maxit=5, verify=0, raise_on_fail=False)
         assert sc.code == gf.GF_ERR_NOCONV and ic.max() == 5
+
+
+@pytest.mark.parametrize("precision", [gf.GF_PREC_FP64, gf.GF_PREC_MIXED])
+@pytest.mark.parametrize("t,nx,ny,nz,nrhs", [
+    (gf.GF_BRICK8, 1, 1, 1, 2), (gf.GF_BRICK8, 3, 3, 3, 9),                # 8 and 64 nodes
+    (gf.GF_BRICK20, 3, 2, 2, 17), (gf.GF_BRICK20, 5, 4, 3, 40),
+    (gf.GF_BRICK8, 22, 22, 22, 33), (gf.GF_BRICK8, 23, 22, 22, 33)])       # 764 and 796 passes
+def test_batched_rows_in_shares(gpu_ctx, t, nx, ny, nz, nrhs, precision):
+    """3D load cases advance with each row's blocks in four shares below the
+    border and in one above it: every column's residual, formed by the
+    thread-per-row product, meets the tolerance the solve reports, and a
+    second solve gives the same bits."""
+    p, K = assembled(gpu_ctx, t, nx, ny, nz)
+    _, R = assembled(gpu_ctx, t, nx, ny, nz)
+    gpu_ctx.tune(R, 0)
+    F = P.random_top_loads(p, nrhs, 5)
+    X, st = gpu_ctx.pcg(K, F, precision=precision)
+    assert st.converged and st.true_relres <= 1.05e-8 and st.fallbacks == 0
+    for k in range(nrhs):
+        assert np.linalg.norm(F[k] - gpu_ctx.spmv(R, X[k])[0]) <= 1.1e-8 * np.linalg.norm(F[k])
+    Y, s2 = gpu_ctx.pcg(K, F, precision=precision)
+    assert np.array_equal(X, Y) and s2.iterations == st.iterations
