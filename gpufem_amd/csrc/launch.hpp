@@ -191,6 +191,18 @@ int spmv_grid(int variant, const BsellView& bs, int nblocks);
 // slice-group variants while the block values (bslots block slots of
 // value_bytes each) stay in the last-level cache, else the variant itself
 int iter_variant(int variant, int64_t bslots, int64_t value_bytes);
+// Whether the iterations of such a matrix run in one workgroup (k_single): its
+// vectors fit the LDS and registers of a CU, and its values are read there
+// sooner (about 120 GB/s past the held ones) than two launches take.  us an
+// iteration, one workgroup / two launches: Q4 4x4 2.3 / 7.5, 40x20 (0.24 MB)
+// 3.5 / 9.4, 64x32 (0.63 MB) 7.2 / 9.8, 64x44 (0.86 MB) 9.7 / 9.7; Q8 30x10
+// 5.5 / 10.0, 32x28 (1.2 MB) 14.2 / 10.1; Brick8 3^3 2.5 / 10.0, 6^3 (0.8 MB)
+// 5.2 / 11.5, 8x8x7 (1.3 MB) 9.7 / 12.0, 11^3 (3.4 MB) 25 / 12.4; Brick20 3x3x2
+// 5.9 / 14.6, 6x5x4 (2.5 MB) 20.5 / 17.4.
+constexpr int64_t single_bytes(int d) { return d == 2 ? 3 << 18 : 5 << 18; }
+template <int D>
+constexpr int kSingleSlices = D == 2 ? 48 : 32;  // of 64 node rows
+bool single_fits(int iter_variant, int64_t n, int64_t bslots, int64_t nslices);
 // bs: the block-sliced view (used by the kBsell variants only; may be null)
 hipError_t launch_spmv(hipStream_t s, int variant, int64_t n, const double* val,
                        const int32_t* col, const int32_t* rownnz, const double* x, double* y,
@@ -207,6 +219,7 @@ struct PcgBuffers {
   int32_t width;
   int variant;       // products outside the iteration (launch_spmv)
   int iter_variant;  // q = K p inside it; a split variant: the two-launch iteration
+  bool single;       // the iterations run in one workgroup (single_fits)
   const double* val;
   const int32_t* col;
   const int32_t* rownnz;
@@ -232,6 +245,11 @@ hipError_t launch_pcg_iteration(hipStream_t s, const PcgBuffers& B, int parity);
 // the same, with events recorded around the SpMV kernel
 hipError_t launch_pcg_iteration_timed(hipStream_t s, const PcgBuffers& B, int parity,
                                       hipEvent_t spmv_start, hipEvent_t spmv_stop);
+// iterations between two looks at the state from the host (even), and of a
+// launch of the single workgroup
+constexpr int kPcgChunk = 32, kSingleChunk = 512;
+// such a chunk, and the state it left
+hipError_t launch_pcg_chunk(hipStream_t s, const PcgBuffers& B);
 // after iterations, the next of which has this parity: the state they left
 hipError_t launch_pcg_check(hipStream_t s, const PcgBuffers& B, int parity);
 // co-resident workgroups for the persistent kernel of this (iteration) variant

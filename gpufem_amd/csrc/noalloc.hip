@@ -41,7 +41,6 @@ constexpr int kMaxDevices = 64;
 std::mutex g_mutex;
 char* g_scratch[kMaxDevices] = {};
 
-constexpr int kChunk = 32;       // iterations between convergence checks, as gf_pcg
 constexpr int kMaxRestarts = 4;  // true-residual restarts, as gf_pcg
 
 }  // namespace
@@ -117,6 +116,7 @@ extern "C" int gf_pcg_noalloc(gf_ctx* ctx, gf_ell* m, const double* b, double* x
   B.width = m->width;
   B.variant = variant;
   B.iter_variant = iter_variant(variant, m->bslots, sizeof(double));
+  B.single = single_fits(B.iter_variant, n, m->bslots, o.bs.nslices);
   B.val = o.val;
   B.col = o.col;
   B.bs = o.bs;
@@ -144,9 +144,7 @@ extern "C" int gf_pcg_noalloc(gf_ctx* ctx, gf_ell* m, const double* b, double* x
     GF_HIP_CHECK(ctx, launch_pcg_setup(ctx->stream, B, use_x0, opts.rtol, opts.maxit - total));
     GF_HIP_CHECK(ctx, read_pcg_state(ctx->stream, B, &h));
     while (!h.done) {
-      for (int it = 0; it < kChunk; ++it)
-        GF_HIP_CHECK(ctx, launch_pcg_iteration(ctx->stream, B, it & 1));
-      GF_HIP_CHECK(ctx, launch_pcg_check(ctx->stream, B, 0));
+      GF_HIP_CHECK(ctx, launch_pcg_chunk(ctx->stream, B));
       GF_HIP_CHECK(ctx, read_pcg_state(ctx->stream, B, &h));
     }
     total += h.it;

@@ -28,7 +28,6 @@ int set_error(gf_ctx* ctx, int code, const std::string& msg);
 
 namespace {
 
-constexpr int kChunk = 32;  // iterations between convergence checks (even)
 constexpr int kMaxRestarts = 4;  // true-residual restarts per right-hand side
 
 double now_ms() {
@@ -50,11 +49,7 @@ hipError_t ensure_graph(gf_ctx* ctx, gf_ell* m, const PcgBuffers& B, int key) {
   hipGraph_t g = nullptr;
   hipError_t e = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) return e;
-  for (int it = 0; it < kChunk; ++it) {
-    e = launch_pcg_iteration(ctx->stream, B, it & 1);
-    if (e != hipSuccess) break;
-  }
-  if (e == hipSuccess) e = launch_pcg_check(ctx->stream, B, 0);
+  e = launch_pcg_chunk(ctx->stream, B);
   hipError_t e2 = hipStreamEndCapture(ctx->stream, &g);
   if (e == hipSuccess) e = e2;
   if (e == hipSuccess) e = hipGraphInstantiate(&P->graph[key], g, nullptr, nullptr, 0);
@@ -295,6 +290,7 @@ PcgBuffers make_buffers(gf_ell* m, const double* dinv) {
   B.width = m->width;
   B.variant = P->variant;
   B.iter_variant = iter_variant(P->variant, m->bslots, sizeof(double));
+  B.single = single_fits(B.iter_variant, m->n, m->bslots, o.bs.nslices);
   B.val = o.val;
   B.col = o.col;
   B.bs = o.bs;
@@ -414,13 +410,11 @@ int run_pcg(gf_ctx* ctx, gf_ell* m, const PcgBuffers& B, int sched, int key, int
     } else {
       GF_HIP_CHECK(ctx, read_pcg_state(ctx->stream, B, h));
       while (!h->done) {
-        if (sched == GF_SCHED_GRAPH) {
+        if (sched == GF_SCHED_GRAPH && !B.single) {
           GF_HIP_CHECK(ctx, ensure_graph(ctx, m, B, B.dinv ? 1 : 0));
           GF_HIP_CHECK(ctx, hipGraphLaunch(P->graph[key], ctx->stream));
         } else {
-          for (int it = 0; it < kChunk; ++it)
-            GF_HIP_CHECK(ctx, launch_pcg_iteration(ctx->stream, B, it & 1));
-          GF_HIP_CHECK(ctx, launch_pcg_check(ctx->stream, B, 0));
+          GF_HIP_CHECK(ctx, launch_pcg_chunk(ctx->stream, B));
         }
         GF_HIP_CHECK(ctx, read_pcg_state(ctx->stream, B, h));
       }
@@ -785,7 +779,8 @@ int gf_profile_pcg(gf_ctx* ctx, gf_ell* m, const double* b, int32_t iters, doubl
   if ((st = prepare_variant(ctx, m, P->variant))) return st;
   GF_HIP_CHECK(ctx, hipMemcpyAsync(P->wb, b, size_t(m->n) * sizeof(double),
                                    hipMemcpyHostToDevice, ctx->stream));
-  const PcgBuffers B = make_buffers(m, m->d_dinv);
+  PcgBuffers B = make_buffers(m, m->d_dinv);
+  B.single = false;  // whose product is no launch of its own
   // rtol 0: every one of the iters iterations runs (unless the residual
   // vanishes exactly)
   GF_HIP_CHECK(ctx, launch_pcg_setup(ctx->stream, B, 0, 0.0, iters));
@@ -796,12 +791,12 @@ int gf_profile_pcg(gf_ctx* ctx, gf_ell* m, const double* b, int32_t iters, doubl
         if (e) (void)hipEventDestroy(e);
     }
   } E;
-  E.ev.assign(2 * kChunk, nullptr);
+  E.ev.assign(2 * kPcgChunk, nullptr);
   for (hipEvent_t& e : E.ev) GF_HIP_CHECK(ctx, hipEventCreate(&e));
   double spmv = 0.0;
   GF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_start, ctx->stream));
   for (int done = 0; done < iters;) {
-    const int c = std::min(kChunk, iters - done);
+    const int c = std::min(kPcgChunk, iters - done);
     for (int k = 0; k < c; ++k)
       GF_HIP_CHECK(ctx, launch_pcg_iteration_timed(ctx->stream, B, (done + k) & 1, E.ev[2 * k],
                                                    E.ev[2 * k + 1]));

@@ -29,7 +29,8 @@
 // chunk of them), with all scalars in a device PcgState, so the host can
 // enqueue or graph-replay chunks of iterations; or one cooperative
 // persistent kernel (k_pcg_persistent, k_split_persistent) with a grid barrier
-// after each of those steps.  Every block reduces the per-block partials in the same fixed
+// after each of those steps.  A small system takes hundreds of iterations in one
+// launch of one workgroup under any schedule (k_single).  Every block reduces the per-block partials in the same fixed
 // order, so all blocks take the same convergence decision and results are
 // bitwise reproducible for a given matrix and variant.  The SpMV kernel may
 // run on a grid of its own (the slice-group variants): k_update reduces its
@@ -374,6 +375,265 @@ __global__ __launch_bounds__(kNT) void k_split_check(PcgBuffers B, int parity) {
     st->rr = rr;
     st->it = st->itv[parity];
     (void)split_goes_on(B, st->it, rr, true);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Small systems in one workgroup (single_fits): `count` iterations a launch, p,
+// q and x in LDS, r and 1 / diagonal in registers, four workgroup barriers an
+// iteration and no other synchronisation (two launches of anything take 7 us).
+// Eight waves take equal runs of the matrix's block slots.  What bounds it is
+// one CU's path to the L2 (64 bytes a clock): each wave keeps the first kHeld
+// slots of its run in registers for the whole launch and streams the others,
+// U in flight at any time and across iterations.  Q4 64x32, 7.2 us an iteration
+// (9.8 in two launches): 2.3 of reductions, barriers and vector steps, 4 of
+// streaming 0.48 MB, the rest of adding; 9.9 with no loads in flight across
+// steps.  A slice that several waves share is summed in wave order, and p.q is
+// taken from whole rows: summed over the waves' partial rows, which cancel, it
+// cost a slender plate 7 of 81 iterations.
+// ---------------------------------------------------------------------------
+constexpr int kSingleWaves = 8;
+
+// v plus the value `ctrl` lanes back (row_shr, row_bcast), in the lanes that
+// have one
+template <int CTRL, int ROWS>
+__device__ inline double dpp_add(double v) {
+  const int64_t b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, int(b), CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, int(b >> 32), CTRL, ROWS, 0xf, false);
+  return v + __longlong_as_double((int64_t(hi) << 32) | uint32_t(lo));
+}
+// a wave's sum, in lane 63: register moves (a shuffle is a trip through the LDS)
+__device__ inline double wave_sum63(double v) {
+  v = dpp_add<0x111, 0xf>(v);
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);
+  return dpp_add<0x143, 0xc>(v);
+}
+template <int D>
+constexpr int kHeld = D == 2 ? 12 : 5;
+
+template <int D>
+__global__ __launch_bounds__(64 * kSingleWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+k_single(PcgBuffers B, int count) {
+  constexpr int W = kSingleWaves, DD = D * D, H = kHeld<D>, U = D == 2 ? 4 : 2;
+  constexpr int SL = kSingleSlices<D>;  // of the matrix, at most
+  constexpr int SW = SL / W;            // of a wave's vector rows
+  static_assert(SL % W == 0, "equal shares");
+  __shared__ double p_[SL * 64 * D];    // by row
+  __shared__ double q_[SL][D][64];      // by position
+  __shared__ double x_[SL][D][64];
+  __shared__ double edge[W][D][64];     // of the slice a wave takes over from the one before
+  __shared__ int64_t s_ptr[SL + 1];
+  __shared__ int s_edge[W];             // its slice, or -1
+  __shared__ double red[3][W];
+  PcgState* st = B.st;
+  if (st->done) return;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int ns = int(B.bs.nslices);
+  for (int s = threadIdx.x; s <= ns; s += 64 * W) s_ptr[s] = B.bs.sptr[s];
+  // this wave's vector rows: lane of slices w, w + W, ...
+  int32_t R[SW];
+  double r[SW][D], d[SW][D];
+#pragma unroll
+  for (int k = 0; k < SW; ++k) {
+    const int s = w + k * W;
+    R[k] = s < ns ? B.bs.perm[s * 64 + lane] : -1;
+    if (s >= ns) continue;
+#pragma unroll
+    for (int e = 0; e < D; ++e) {
+      const int64_t i = int64_t(D) * (R[k] >= 0 ? R[k] : 0) + e;
+      r[k][e] = R[k] >= 0 ? B.r[i] : 0.0;
+      d[k][e] = B.dinv && R[k] >= 0 ? B.dinv[i] : 1.0;
+      x_[s][e][lane] = R[k] >= 0 ? B.x[i] : 0.0;
+      q_[s][e][lane] = 0.0;  // slices without blocks
+      if (R[k] >= 0) p_[i] = B.p[i];
+    }
+  }
+  __syncthreads();
+  // this wave's run of block slots, and the slice it begins in
+  const int64_t T = s_ptr[ns], b0 = T * w / W, b1 = T * (w + 1) / W;
+  int first = 0;
+  while (first < ns && s_ptr[first + 1] <= b0) ++first;
+  if (lane == 0) s_edge[w] = first < ns && b1 > b0 && s_ptr[first] < b0 ? first : -1;
+  double hv[H][DD];
+  int32_t hc[H];
+#pragma unroll
+  for (int k = 0; k < H; ++k) {
+    if (b0 + k < b1) {
+      load_block<D, double, false>(B.val, b0 + k, lane, hv[k]);
+      hc[k] = B.col[(b0 + k) * 64 + lane];
+    }
+  }
+  // the streamed ones: U in flight
+  const int64_t bs0 = b0 + H;
+  double sv[U][DD];
+  int32_t sc[U];
+  auto fetch = [&](int u, int64_t b) {
+    b = b < b1 ? b : b1 - 1;
+    load_block<D, double, false>(B.val, b, lane, sv[u]);
+    sc[u] = B.col[b * 64 + lane];
+  };
+  if (bs0 < b1) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) fetch(u, bs0 + u);
+  }
+  __syncthreads();  // s_edge
+  uint32_t edges[SW];  // waves whose edge belongs to this wave's slices
+#pragma unroll
+  for (int k = 0; k < SW; ++k) {
+    edges[k] = 0;
+#pragma unroll
+    for (int j = 1; j < W; ++j)
+      if (s_edge[j] == w + k * W) edges[k] |= 1u << j;
+    edges[k] = __builtin_amdgcn_readfirstlane(edges[k]);
+  }
+  double rho = st->rho[0], rr = st->rr;
+  int it = st->it, status = GF_OK, done = 0;
+  const int maxit = st->maxit;
+  const double tol2 = st->rtol2 * st->bnorm2;
+  // sum of a value over the workgroup, the same in every thread
+  auto leave = [&](int j, double v) {
+    v = wave_sum63(v);
+    if (lane == 63) red[j][w] = v;
+  };
+  auto total = [&](int j) {
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < W; ++k) t += red[j][k];
+    return t;
+  };
+  for (int left = count; left > 0; --left) {
+    __syncthreads();  // p
+    double acc[D];
+#pragma unroll
+    for (int e = 0; e < D; ++e) acc[e] = 0.0;
+    int s = first;
+    int64_t end = first < ns ? s_ptr[first + 1] : 0;
+    // a slice is summed, or this wave's part of it
+    auto flush = [&]() {
+      double* out = s_ptr[s] >= b0 ? &q_[s][0][lane] : &edge[w][0][lane];
+#pragma unroll
+      for (int e = 0; e < D; ++e) {
+        out[e * 64] = acc[e];
+        acc[e] = 0.0;
+      }
+    };
+    auto next = [&](int64_t b) {
+      if (b < end) return;
+      flush();
+      do end = s_ptr[++s + 1];
+      while (end <= b);
+    };
+    auto add = [&](const double* v, int32_t c) {
+#pragma unroll
+      for (int f = 0; f < D; ++f) {
+        const double xv = p_[D * c + f];
+#pragma unroll
+        for (int e = 0; e < D; ++e) acc[e] += v[e * D + f] * xv;
+      }
+    };
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+      if (b0 + k < b1) {
+        next(b0 + k);
+        add(hv[k], hc[k]);
+      }
+    }
+    for (int64_t b = bs0; b < b1; b += U) {
+      // the buffer of a slot takes the one U further on as soon as it is used
+      // up, at the end of the run the first ones of the next iteration
+      const int64_t ahead = b + U < b1 ? b + U : bs0;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (b + u < b1) {
+          next(b + u);
+          add(sv[u], sc[u]);
+        }
+        fetch(u, ahead + u);
+      }
+    }
+    if (b1 > b0) flush();
+    __syncthreads();
+    // p.q from the whole sums of a row, which the residual takes too
+    double pq = 0.0;
+#pragma unroll
+    for (int k = 0; k < SW; ++k) {
+      const int sk = w + k * W;
+      if (R[k] < 0) continue;
+#pragma unroll
+      for (int e = 0; e < D; ++e) {
+        double q = q_[sk][e][lane];
+        if (edges[k]) {
+          for (uint32_t m = edges[k]; m; m &= m - 1) q += edge[__builtin_ctz(m)][e][lane];
+          q_[sk][e][lane] = q;
+        }
+        pq += p_[D * R[k] + e] * q;
+      }
+    }
+    leave(0, pq);
+    __syncthreads();
+    pq = total(0);
+    if (!(pq > 0.0)) {
+      status = GF_ERR_BREAKDOWN;
+      done = 1;
+      break;
+    }
+    const double alpha = rho / pq;
+    double rz = 0.0;
+    rr = 0.0;
+#pragma unroll
+    for (int k = 0; k < SW; ++k) {
+      const int sk = w + k * W;
+      if (R[k] < 0) continue;
+#pragma unroll
+      for (int e = 0; e < D; ++e) {
+        x_[sk][e][lane] += alpha * p_[D * R[k] + e];
+        r[k][e] -= alpha * q_[sk][e][lane];
+        rz += r[k][e] * (d[k][e] * r[k][e]);
+        rr += r[k][e] * r[k][e];
+      }
+    }
+    leave(1, rz);
+    leave(2, rr);
+    __syncthreads();
+    rz = total(1);
+    rr = total(2);
+    ++it;
+    if (rr <= tol2 || it >= maxit) {
+      done = 1;
+      break;
+    }
+    const double beta = rz / rho;
+    rho = rz;
+#pragma unroll
+    for (int k = 0; k < SW; ++k) {
+      if (R[k] < 0) continue;
+#pragma unroll
+      for (int e = 0; e < D; ++e)
+        p_[D * R[k] + e] = d[k][e] * r[k][e] + beta * p_[D * R[k] + e];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < SW; ++k) {
+    if (R[k] < 0) continue;
+#pragma unroll
+    for (int e = 0; e < D; ++e) {
+      const int64_t i = int64_t(D) * R[k] + e;
+      B.x[i] = x_[w + k * W][e][lane];
+      B.r[i] = r[k][e];
+      B.p[i] = p_[i];
+    }
+  }
+  if (threadIdx.x == 0) {
+    st->rho[0] = rho;
+    st->rr = rr;
+    st->it = it;
+    st->status = status;
+    st->done = done;
   }
 }
 
@@ -834,9 +1094,9 @@ hipError_t launch_pcg_setup(hipStream_t s, const PcgBuffers& B, int use_x0, doub
     e = launch_spmv(s, B.variant, B.n, B.val, B.col, B.rownnz, B.x, B.q, 1, &B.bs);
     if (e != hipSuccess) return e;
   }
-  if (B.iter_variant == kSplit2)
+  if (!B.single && B.iter_variant == kSplit2)
     hipLaunchKernelGGL(k_pcg_init<2>, dim3(B.nblocks), dim3(kNT), 0, s, B, use_x0);
-  else if (B.iter_variant == kSplit3)
+  else if (!B.single && B.iter_variant == kSplit3)
     hipLaunchKernelGGL(k_pcg_init<3>, dim3(B.nblocks), dim3(kNT), 0, s, B, use_x0);
   else
     hipLaunchKernelGGL(k_pcg_init<1>, dim3(B.nblocks), dim3(kNT), 0, s, B, use_x0);
@@ -878,9 +1138,34 @@ hipError_t launch_updates(hipStream_t s, const PcgBuffers& B, int parity) {
 }
 }  // namespace
 
+bool single_fits(int iter_variant, int64_t n, int64_t bslots, int64_t nslices) {
+  if (!is_split_variant(iter_variant)) return false;
+  const int d = iter_variant == kSplit2 ? 2 : 3;
+  return nslices <= (d == 2 ? kSingleSlices<2> : kSingleSlices<3>) &&
+         n <= nslices * 64 * d && bslots * 64 * d * d * int64_t(sizeof(double)) <= single_bytes(d);
+}
+
+namespace {
+hipError_t launch_single(hipStream_t s, const PcgBuffers& B, int count) {
+  const dim3 blk(64 * kSingleWaves);
+  if (B.iter_variant == kSplit2)
+    hipLaunchKernelGGL(k_single<2>, dim3(1), blk, 0, s, B, count);
+  else
+    hipLaunchKernelGGL(k_single<3>, dim3(1), blk, 0, s, B, count);
+  return hipGetLastError();
+}
+}  // namespace
+
 hipError_t launch_pcg_iteration(hipStream_t s, const PcgBuffers& B, int parity) {
   const hipError_t e = launch_product(s, B, parity);
   return e != hipSuccess ? e : launch_updates(s, B, parity);
+}
+
+hipError_t launch_pcg_chunk(hipStream_t s, const PcgBuffers& B) {
+  if (B.single) return launch_single(s, B, kSingleChunk);
+  hipError_t e = hipSuccess;
+  for (int it = 0; it < kPcgChunk && e == hipSuccess; ++it) e = launch_pcg_iteration(s, B, it & 1);
+  return e != hipSuccess ? e : launch_pcg_check(s, B, 0);
 }
 
 hipError_t launch_pcg_check(hipStream_t s, const PcgBuffers& B, int parity) {
@@ -924,6 +1209,7 @@ int persistent_blocks(int variant, int num_cu) {
 }
 
 hipError_t launch_pcg_persistent(hipStream_t s, const PcgBuffers& B, void* barrier, int num_cu) {
+  if (B.single) return launch_single(s, B, INT32_MAX);
   GridBarrier* bar = static_cast<GridBarrier*>(barrier);
   hipLaunchKernelGGL(k_barrier_reset, dim3(1), dim3(64), 0, s, bar);
   hipError_t e = hipGetLastError();

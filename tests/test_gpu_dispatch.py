@@ -139,3 +139,34 @@ def test_batched_rows_in_shares(gpu_ctx, t, nx, ny, nz, nrhs, precision):
         assert np.linalg.norm(F[k] - gpu_ctx.spmv(R, X[k])[0]) <= 1.1e-8 * np.linalg.norm(F[k])
     Y, s2 = gpu_ctx.pcg(K, F, precision=precision)
     assert np.array_equal(X, Y) and s2.iterations == st.iterations
+
+
+@pytest.mark.parametrize("t,nx,ny,nz", [
+    (gf.GF_Q4, 1, 1, 0), (gf.GF_Q4, 7, 7, 0), (gf.GF_Q4, 15, 7, 0),      # 1, 1 and 2 slices
+    (gf.GF_Q4, 47, 38, 0), (gf.GF_Q4, 63, 41, 0), (gf.GF_Q4, 63, 42, 0),  # 42 slices is the last
+    (gf.GF_Q8, 21, 13, 0), (gf.GF_BRICK8, 1, 1, 1), (gf.GF_BRICK8, 7, 7, 7),
+    (gf.GF_BRICK20, 2, 1, 1), (gf.GF_BRICK20, 4, 4, 3)])
+@pytest.mark.parametrize("sched", [gf.GF_SCHED_KERNELS, gf.GF_SCHED_PERSISTENT])
+def test_small_system_in_one_workgroup(gpu_ctx, t, nx, ny, nz, sched):
+    """Systems at the edges of the single workgroup's range: the residual
+    formed by the thread-per-row product meets the tolerance, with and without
+    the preconditioner and an initial guess; more iterations than one launch
+    takes, an iteration limit inside a launch and a finished state are the
+    limits' own."""
+    p, K = assembled(gpu_ctx, t, nx, ny, nz)
+    _, R = assembled(gpu_ctx, t, nx, ny, nz)
+    gpu_ctx.tune(R, 0)
+    f = p.f
+    x, st = gpu_ctx.pcg(K, f, schedule=sched)
+    assert st.converged and st.true_relres <= 1.05e-8
+    assert np.linalg.norm(f - gpu_ctx.spmv(R, x)[0]) <= 1.1e-8 * np.linalg.norm(f)
+    y, s2 = gpu_ctx.pcg(K, f)
+    assert np.array_equal(x, y) and s2.iterations == st.iterations
+    _, s3 = gpu_ctx.pcg(K, f, x0=x, rtol=1.1e-8, schedule=sched)
+    assert s3.iterations == 0
+    _, s4 = gpu_ctx.pcg(K, f, rtol=1e-300, maxit=700, schedule=sched, verify=0, raise_on_fail=False)
+    assert s4.iterations == 700 or s4.code == gf.GF_ERR_BREAKDOWN
+    _, s5 = gpu_ctx.pcg(K, f, maxit=3, schedule=sched, raise_on_fail=False)
+    assert s5.iterations == min(3, st.iterations)
+    z, s6 = gpu_ctx.pcg(K, np.zeros_like(f), schedule=sched)
+    assert s6.iterations == 0 and not z.any()
