@@ -449,17 +449,38 @@ struct GArgs {
   const double* geom;
 };
 
+// nonzero where a byte of w equals the same byte of another lane of the eight
+// (lanes 8 i .. 8 i + 7) this one belongs to
+__device__ inline uint32_t same_byte8(uint32_t w) {
+  auto eq = [&](uint32_t o) {
+    const uint32_t x = w ^ o;
+    return (x - 0x01010101u) & ~x & 0x80808080u;
+  };
+  auto quad = [&](uint32_t v) {  // the other three lanes of the quad
+    return eq(uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0xb1, 0xf, 0xf, false))) |
+           eq(uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x4e, 0xf, 0xf, false))) |
+           eq(uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x1b, 0xf, 0xf, false)));
+  };
+  const uint32_t m = uint32_t(__builtin_amdgcn_mov_dpp(int(w), 0x141, 0xf, 0xf, false));  // lane 7 - i
+  return quad(w) | eq(m) | quad(m);
+}
+
 // A unit is RPT rows of one node (UPN units per node).  LPU lanes share a
 // unit: lane j of the unit takes the node's incidences j, j + LPU, ... and the
-// LPU lanes add their element's rows into the unit's LDS accumulators in LPU
-// masked phases, so every accumulator receives the elements in ascending
-// incidence order when the neighbours form one chunk (BCH = NEN).  With
-// smaller chunks the LPU elements of a trip add chunk by chunk, and a slot
-// that is neighbour b of one element and a later-chunk neighbour of an
-// earlier one receives them out of order: the sums then depend on LPU in
-// their last bits (the same configuration gives the same bits).  UPW units per 64-lane
-// workgroup: LPU > 1 divides the LDS per workgroup by LPU and lets more
-// wavefronts share a CU.
+// lanes add their element's rows into the unit's LDS accumulators.
+// Eight lanes (3D node units): neighbour b of all of them in one step where no
+// two lanes' neighbours b are one node (same_byte8 of the slot maps: so on any
+// mesh whose elements are numbered alike), every slot receiving its terms in
+// ascending b.  Otherwise LPU masked phases, one lane of each unit at a time:
+// the elements in ascending incidence order when the neighbours form one chunk
+// (BCH = NEN); with smaller chunks the LPU elements of a trip add chunk by
+// chunk, and a slot that is neighbour b of one element and a later-chunk
+// neighbour of an earlier one receives them out of order: the sums then depend
+// on LPU in their last bits.  The same configuration and mesh give the same bits
+// either way.  The phases kept 8 of 64 lanes busy: Brick8 101x90x88 1.72 -> 1.42
+// ms, Brick20 30x33x28 over its element tensors 1.11 -> 0.99.
+// UPW units per 64-lane workgroup: LPU > 1 divides the LDS per workgroup by LPU
+// and lets more wavefronts share a CU.
 // With RPT == DIM (every row of the node in one unit) the lane forms the
 // products T_pq = sum_g (w detJ E dNa/dx_p)(dNb/dx_q) per neighbour b and the
 // elastic combinations once per element; the element's nodes b are taken BCH
@@ -472,13 +493,16 @@ struct GArgs {
 // SRC 0's bitwise).
 template <int DIM, int NEN, int NGP, int MAXS, int RPT, int LPU, int UPW, int BCH, int GPU = 1,
           int SRC = 0>
-__global__ __launch_bounds__(64) void k_assemble_gather(GArgs ga) {
+__global__ __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(DIM == 3 && NEN == 8 ? 2 : 1))) void
+k_assemble_gather(GArgs ga) {
   static_assert(LPU * UPW <= 64, "a workgroup is one wavefront");
   static_assert(SRC != 1 || (RPT == DIM && DIM == 3), "element tensors: 3D node units");
   static_assert(SRC != 2 || RPT == DIM, "stored geometry: node units");
   static_assert(NEN % BCH == 0 && (RPT == DIM || BCH == NEN), "neighbour chunks");
   constexpr int UPN = DIM / RPT;  // units per node
   constexpr int ACC = MAXS * RPT * DIM;
+  constexpr bool kApart = LPU == 8 && NEN % 4 == 0;
   __shared__ double s_acc[ACC * UPW];
   const KArgs& a = ga.k;
   const int lu = threadIdx.x / LPU;  // unit of this lane inside the workgroup
@@ -502,6 +526,24 @@ __global__ __launch_bounds__(64) void k_assemble_gather(GArgs ga) {
     }
     for (int t = 0; t < trips; ++t) {
       const int64_t kk = k0 + int64_t(t) * LPU + lj;
+      bool apart = false;
+      if constexpr (kApart) {
+        // (a lane without an element: a byte that is no slot and no lane's but its own)
+        uint32_t w[NEN / 4];
+#pragma unroll
+        for (int i = 0; i < NEN / 4; ++i) w[i] = (0x80u + lj) * 0x01010101u;
+        if (kk < k1) {
+          const int32_t packed = ga.n2e[kk];
+          const uint32_t* sw = reinterpret_cast<const uint32_t*>(
+              a.slot + (int64_t(packed >> 5) * NEN + (packed & 31)) * NEN);
+#pragma unroll
+          for (int i = 0; i < NEN / 4; ++i) w[i] = sw[i];
+        }
+        uint32_t same = 0;
+#pragma unroll
+        for (int i = 0; i < NEN / 4; ++i) same |= same_byte8(w[i]);
+        apart = !__any(int(same));
+      }
       if (kk >= k1) continue;  // this lane's share of the node is done
       const int32_t packed = ga.n2e[kk];
       const int64_t e = packed >> 5;
@@ -645,6 +687,18 @@ __global__ __launch_bounds__(64) void k_assemble_gather(GArgs ga) {
         int sb[BCH];
 #pragma unroll
         for (int b = 0; b < BCH; ++b) sb[b] = sl[c0 + b];
+        if (apart) {
+#pragma unroll
+          for (int b = 0; b < BCH; ++b) {
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int r = 0; r < RPT; ++r)
+#pragma unroll
+              for (int j = 0; j < DIM; ++j)
+                s_acc[((sb[b] * RPT + r) * DIM + j) * UPW + lu] += kl[b][r][j];
+          }
+          continue;
+        }
 #pragma unroll
         for (int p = 0; p < LPU; ++p) {
           if constexpr (LPU > 1) __builtin_amdgcn_wave_barrier();
@@ -1061,13 +1115,14 @@ hipError_t launch_gather_cfg(hipStream_t s, const GArgs& g) {
 //      per node: 0.86 ms, 43 KB of LDS per workgroup, 1 wavefront per SIMD).
 //  Brick8: node units, 8 lanes per node, 8 nodes per workgroup (15.5 KB of
 //      LDS: up to 8 one-wave workgroups per CU, as the registers allow; 4 x 16
-//      with 31 KB fits 5: 4.18 ms), neighbours in chunks of 4 (all 8 at once:
-//      6.0 ms), Gauss-point loop unrolled by 2 (the table loads of two points
-//      batched: 4.38 -> 4.18 ms at 4 x 16; by 4: 4.75 ms; unrolled by 1 at
-//      8 x 8: 4.29 ms; the 2D and Brick20 kernels gain nothing or lose):
-//      128^3 4.06-4.08 ms; row units (one row per unit, each element's
-//      geometry once per row): 6.3-6.6 ms with 2 lanes per row, 9.7 ms with
-//      one lane per row.
+//      with 31 KB fits 5), all 8 neighbours at once (the geometry once per
+//      incidence) at two waves per SIMD, Gauss-point loop rolled: 101x90x88
+//      1.36 ms, over the stored geometry 1.56; neighbours in chunks of 4 with
+//      two points unrolled 1.42 and 1.87, two points unrolled and 8 neighbours
+//      1.8, three waves 1.6 or more.  Then 54 % of the cycles issue vector
+//      instructions (FP64 mostly) and 36 % wait for loads.  Row units (one row
+//      per unit, each element's geometry once per row) took 1.6 times the node
+//      units with 2 lanes per row, 2.4 with one lane per row.
 //  Brick20: row units, 4 lanes per row (256 VGPRs + AGPRs): 48^3 8.1-8.7 ms;
 //      node units need chunks of at most 4 neighbours for their registers and
 //      recompute the 20-node geometry per chunk (10.8-20.5 ms).
@@ -1195,7 +1250,7 @@ hipError_t launch_assembly_geom(hipStream_t s, const AssemblyArgs& a, double* ge
                 : launch_geom<2, 8, 4, 21, 2, 30, 8, 1>(s, a, geom);
     case GF_BRICK8:
       return g3 ? launch_geom<3, 8, 27, 27, 8, 8, 4, 2>(s, a, geom)
-                : launch_geom<3, 8, 8, 27, 8, 8, 4, 2>(s, a, geom);
+                : launch_geom<3, 8, 8, 27, 8, 8, 8, 1>(s, a, geom);
     case GF_BRICK20:
       return g3 ? launch_geom<3, 20, 27, 81, 8, 8, 10, 1>(s, a, geom)
                 : launch_geom<3, 20, 8, 81, 8, 8, 10, 1>(s, a, geom);
@@ -1214,7 +1269,7 @@ hipError_t launch_assembly_gather(hipStream_t s, const AssemblyArgs& a) {
     case GF_Q8: return g3 ? launch_gather2<8, 9, 21>(s, g) : launch_gather2<8, 4, 21>(s, g);
     case GF_BRICK8:
       return g3 ? launch_gather_cfg<3, 8, 27, 27, 3, 8, 8, 4, 2>(s, g)
-                : launch_gather_cfg<3, 8, 8, 27, 3, 8, 8, 4, 2>(s, g);
+                : launch_gather_cfg<3, 8, 8, 27, 3, 8, 8, 8, 1>(s, g);
     case GF_BRICK20:
       return g3 ? launch_gather_cfg<3, 20, 27, 81, 1, 4, 16, 20>(s, g)
                 : launch_gather_cfg<3, 20, 8, 81, 1, 4, 16, 20>(s, g);

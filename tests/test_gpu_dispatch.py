@@ -170,3 +170,41 @@ def test_small_system_in_one_workgroup(gpu_ctx, t, nx, ny, nz, sched):
     assert s5.iterations == min(3, st.iterations)
     z, s6 = gpu_ctx.pcg(K, np.zeros_like(f), schedule=sched)
     assert s6.iterations == 0 and not z.any()
+
+
+def turned(conn, coords):
+    """Every third element's numbering turned by 90 degrees about z."""
+    X = coords[conn[0] - 1]
+    nat = np.rint(2 * (X - X.min(0)) / np.ptp(X, axis=0) - 1).astype(int)
+    at = {tuple(v): k for k, v in enumerate(nat)}
+    turn = [at[(-v[1], v[0], v[2])] for v in nat]
+    out = conn.copy()
+    out[::3] = conn[::3][:, turn]
+    return out
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("t,nx,ny,nz,variant", [
+    (gf.GF_BRICK8, 1, 1, 1, 3), (gf.GF_BRICK8, 3, 5, 2, 3), (gf.GF_BRICK8, 7, 4, 4, 4),
+    (gf.GF_BRICK20, 1, 1, 1, 2), (gf.GF_BRICK20, 3, 2, 4, 2), (gf.GF_BRICK20, 3, 2, 4, 4)])
+def test_gather_adds_alike_and_turned_elements(gpu_ctx, t, nx, ny, nz, variant, mixed):
+    """The node gathers on elements numbered alike (no two elements around a
+    node share a neighbour's number) and on a mesh where some do: against the
+    oracle to 1e-12 of the largest value, and the same bits twice."""
+    g = gf.Grid(t, nx, ny, nz)
+    conn, coords = g.fill()
+    conn = np.asarray(conn).reshape(-1, 8 if t == gf.GF_BRICK8 else 20)
+    if mixed:
+        conn = turned(conn, coords)
+    coords = coords + 0.05 * np.random.default_rng(3).uniform(-1, 1, coords.shape)
+    ng = 3 if t == gf.GF_BRICK20 else 2
+    mesh = gpu_ctx.upload_mesh(t, ng, conn, coords, 210000.0, 0.3)
+    K = gpu_ctx.symbolic(mesh)
+    gpu_ctx.assemble_tune(mesh, K, variant)
+    gpu_ctx.assemble(mesh, K)
+    val = gpu_ctx.download(K)[0]
+    gpu_ctx.assemble(mesh, K)
+    assert np.array_equal(val, gpu_ctx.download(K)[0])
+    Ko, _ = O.assemble(g.dim, ng, conn, coords, 210000.0, 0.3, skip_zero=False)
+    ov = Ko.export(Ko.max_rownnz())[0]
+    assert np.abs(val - ov).max() <= 1e-12 * np.abs(ov).max()
