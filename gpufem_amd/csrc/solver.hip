@@ -1217,10 +1217,16 @@ hipError_t launch_pcg_persistent(hipStream_t s, const PcgBuffers& B, void* barri
   PcgBuffers Bc = B;
   void* args[] = {&Bc, &bar};
   // the split kernels play the logical workgroups of both steps in turn; the
-  // others' vector steps take exactly the grid of the kernel schedule
+  // others' vector steps take exactly the grid of the kernel schedule.  Every
+  // workgroup makes the barrier longer (1024 of them: 43 us), so a workgroup for
+  // 1024 rows, from a quarter to all of the CUs; us an iteration against as many
+  // as are co-resident, Q8 201x67 30 / 72, 512x256 119 / 154, Brick8 64x32x32
+  // 58 / 121.
   int nb = B.nblocks;
   if (is_split_variant(B.iter_variant)) {
-    nb = std::min(std::max(B.nblocks, B.spmv_grid), persistent_blocks(B.iter_variant, num_cu));
+    nb = std::min(std::max(num_cu / 4, B.nblocks), num_cu);
+    nb = std::min(nb, std::min(std::max(B.nblocks, B.spmv_grid),
+                               persistent_blocks(B.iter_variant, num_cu)));
     if (nb < 1) return hipErrorInvalidConfiguration;
   }
   const dim3 g(nb), blk(kNT);
