@@ -27,7 +27,7 @@ struct MultiState {
   int32_t col_done[S];  // 1: converged (or empty) column
   int32_t col_status[S];
   int32_t it, done, status, maxit;
-  uint32_t arrived;  // workgroups of k_b_beta finished in this iteration
+  int32_t arrived;  // workgroups of k_b_beta finished in this iteration
   double rtol2;
 };
 
@@ -209,33 +209,27 @@ __global__ __launch_bounds__(kNT) void k_b_beta(MultiBuffers B, int nb) {
   if (st->done) return;
   __shared__ double sh[kNT];
   const int k = blockIdx.x;
-  const double rz = reduce_column(B.part2, nb, k, sh);
-  const double rr = reduce_column(B.part2, nb, S + k, sh);
+  double rz, rr;
+  reduce_column2(B.part2, nb, k, S + k, &rz, &rr, sh);
   if (threadIdx.x == 0) {
     const int it = st->it + 1;
     double beta = 0.0;
-    if (!st->col_done[k]) {
+    int done = st->col_done[k];
+    if (!done) {
       beta = rz / st->rho[k];
       st->rho[k] = rz;
       st->rr[k] = rr;
       st->col_it[k] = it;
       if (rr <= st->rtol2 * st->bnorm2[k] || it >= st->maxit) {
-        st->col_done[k] = 1;
+        st->col_done[k] = done = 1;
         beta = 0.0;
       }
     }
     st->beta[k] = beta;
-    // publish this column's state before arriving; the last arrival reads
-    // every column's
-    __threadfence();
-    if (atomicAdd(&st->arrived, 1u) == S - 1) {
-      __threadfence();
-      int all = 1;
-      for (int j = 0; j < S; ++j)
-        all &= __hip_atomic_load(&st->col_done[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      st->arrived = 0;
+    int ndone;
+    if (arrive<S>(&st->arrived, done, &ndone)) {
       st->it = it;
-      if (all) st->done = 1;
+      if (ndone == S) st->done = 1;
     }
   }
 }

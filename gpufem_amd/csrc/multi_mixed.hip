@@ -242,8 +242,8 @@ __global__ __launch_bounds__(kNT) void k_mm_decide(MixedMultiBuffers B, int nb) 
   if (st->done) return;
   __shared__ double sh[kNT];
   const int k = blockIdx.x;
-  const double rz = reduce_column(B.part2, nb, k, sh);
-  const double rr = reduce_column(B.part2, nb, S + k, sh);
+  double rz, rr;
+  reduce_column2(B.part2, nb, k, S + k, &rz, &rr, sh);
   if (threadIdx.x == 0) {
     st->rz_new[k] = rz;
     st->rr_rec[k] = rr;
@@ -266,14 +266,13 @@ __global__ __launch_bounds__(kNT) void k_mm_beta(MixedMultiBuffers B, int nb) {
   const int k = blockIdx.x;
   const int refreshed = st->any_refresh;
   double rz2 = 0.0, rr2 = 0.0;
-  if (refreshed) {  // the same value in every thread of every workgroup
-    rz2 = reduce_column(B.part3, nb, k, sh);
-    rr2 = reduce_column(B.part3, nb, S + k, sh);
-  }
+  if (refreshed)  // the same value in every thread of every workgroup
+    reduce_column2(B.part3, nb, k, S + k, &rz2, &rr2, sh);
   if (threadIdx.x == 0) {
     const int it = st->it + 1;
     double beta = 0.0;
-    if (!st->col_done[k]) {
+    int done = st->col_done[k];
+    if (!done) {
       double rz = st->rz_new[k];
       bool stalled = false;
       if (st->col_refresh[k]) {
@@ -293,32 +292,26 @@ __global__ __launch_bounds__(kNT) void k_mm_beta(MixedMultiBuffers B, int nb) {
         B.hist[2 * (int64_t(S) * (it - 1) + k) + 1] = rz / st->rho[k];
       }
       if (st->col_refresh[k] && st->rr_true[k] <= st->rtol2 * st->bnorm2[k]) {
-        st->col_done[k] = 1;
+        done = 1;
       } else if (stalled) {
-        st->col_done[k] = 1;
+        done = 1;
         st->col_status[k] = kMixedStalled;
       } else if (it >= st->maxit) {
-        st->col_done[k] = 1;
+        done = 1;
         st->col_status[k] = GF_ERR_NOCONV;
       } else {
         beta = rz / st->rho[k];
         st->rho[k] = rz;
       }
+      st->col_done[k] = done;
     }
     st->beta[k] = beta;
     st->col_refresh[k] = 0;
-    // publish this column's state before arriving; the last arrival reads
-    // every column's
-    __threadfence();
-    if (atomicAdd(&st->arrived, 1) == S - 1) {
-      __threadfence();
-      int all = 1;
-      for (int j = 0; j < S; ++j)
-        all &= __hip_atomic_load(&st->col_done[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      st->arrived = 0;
+    int ndone;
+    if (arrive<S>(&st->arrived, done, &ndone)) {
       st->it = it;
       st->any_refresh = 0;
-      if (all) st->done = 1;
+      if (ndone == S) st->done = 1;
     }
   }
 }
