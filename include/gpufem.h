@@ -322,7 +322,8 @@ int gf_pcg(gf_ctx* ctx, gf_ell* m, const double* b, double* x, int32_t nrhs,
  * the fastest.  gf_pcg does this on first use, but takes 9/10 untimed for a
  * mesh matrix that stays in the last-level cache: there its iteration is two
  * launches, several waves share a slice, and the sums agree with the variant's
- * products to rounding.  ms_per_variant (may be NULL)
+ * products to rounding (a small system: one launch of one workgroup for many
+ * iterations, whatever the schedule).  ms_per_variant (may be NULL)
  * receives GF_SPMV_VARIANTS averages (-1 for variants that do not fit).  No
  * reference counterpart; it plays the role of SetOclStrategy /
  * SetOclLocalSize (src/SPRmatrix/SPRmatrix.h:110-121) chosen by measurement
@@ -339,7 +340,7 @@ int gf_ell_tune(gf_ctx* ctx, gf_ell* m, int32_t force_variant, double* ms_per_va
 int gf_profile_spmv(gf_ctx* ctx, gf_ell* m, int32_t nrep, double* ms_avg);
 
 /* Runs iters Jacobi-PCG iterations from x = 0 for the right-hand side b
- * (host array of n) with the three-launch schedule, HIP events around each
+ * (host array of n) with the two- or three-launch schedule, HIP events around each
  * iteration's SpMV kernel: ms_spmv is that kernel's average duration inside
  * the solve (p freshly rewritten by the previous iteration, as in gf_pcg),
  * ms_iteration the average wall time of one iteration including the event
