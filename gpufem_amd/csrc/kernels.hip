@@ -1204,8 +1204,8 @@ hipError_t launch_assembly_tensors(hipStream_t s, const AssemblyArgs& a, double*
       return g3 ? launch_tensors<8, 27, 27, 4, 16, 8>(s, a, tens)
                 : launch_tensors<8, 8, 27, 4, 16, 8>(s, a, tens);
     case GF_BRICK20:
-      // gather phase: 8 lanes x 8 nodes, neighbours 10 at a time (48^3: 4.19 ms;
-      // chunks of 4/5: 4.22-4.23, 16 lanes x 4 nodes: 4.40-4.49, 4 x 8: 4.46)
+      // gather phase: 8 lanes x 8 nodes, neighbours 10 at a time (30x33x28 with the
+      // tensors 0.99 ms; 5 at a time 1.01, 4 nodes a workgroup 1.04-1.08)
       return g3 ? launch_tensors<20, 27, 81, 8, 8, 10>(s, a, tens)
                 : launch_tensors<20, 8, 81, 8, 8, 10>(s, a, tens);
     default: return hipErrorInvalidValue;
