@@ -19,15 +19,17 @@ namespace {
 thread_local std::string g_last_error;
 }
 
+// A failed HIP call is reported here and forgotten by the runtime: later
+// successes do not reset its error, so the hipGetLastError after the next
+// launch, in whatever call follows, would report it again.
 int set_error(gf_ctx* ctx, int code, const std::string& msg) {
+  if (code == GF_ERR_HIP || code == GF_ERR_NOMEM) (void)hipGetLastError();
   g_last_error = msg;
   if (ctx) ctx->err = msg;
   return code;
 }
 int set_error(const gf_ctx* ctx, int code, const std::string& msg) {
-  g_last_error = msg;
-  if (ctx) const_cast<gf_ctx*>(ctx)->err = msg;
-  return code;
+  return set_error(const_cast<gf_ctx*>(ctx), code, msg);
 }
 
 namespace {

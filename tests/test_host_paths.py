@@ -1,0 +1,65 @@
+"""The host code of libgpufem over a stand-in for the HIP runtime
+(tests/cpp/fake_hip.cpp), no GPU: what it does when an allocation fails and
+which kernels it picks.  Each case runs in a process of its own, where the
+stand-in is loaded before the library."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = """
+import ctypes as C, sys
+fake = C.CDLL(%r, mode=C.RTLD_GLOBAL)
+fake.fake_fail_at.argtypes = [C.c_int64]
+fake.fake_memory.argtypes = [C.c_int64, C.c_int64]
+fake.fake_cost.argtypes = [C.c_char_p, C.c_double]
+fake.fake_log.restype = C.c_char_p
+for f in ("live", "live_bytes", "mallocs", "h2d"):
+    getattr(fake, "fake_" + f).restype = C.c_int64
+sys.path.insert(0, %r)
+import numpy as np
+import gpufem_amd as gf
+from gpufem_amd import problems as P
+ctx = gf.Context(0)
+
+def kernels():
+    return [k for k in fake.fake_log().decode().split("\\n") if k]
+
+def launched(name):
+    return any(name in k for k in kernels())
+
+def mesh_of(p):
+    return ctx.upload_mesh(p.elem_type, p.ngauss, p.conn, p.coords, p.E, p.nu)
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-fPIC", "-shared",
+                    "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(ROOT, "tests", "cpp", "fake_hip.cpp"), "-o", so], check=True)
+
+    def go(body):
+        out = subprocess.run([sys.executable, "-c", PRELUDE % (so, ROOT) + body],
+                             capture_output=True, text=True, timeout=300)
+        assert out.returncode == 0, out.stdout + out.stderr
+    return go
+
+
+def test_a_reported_failure_is_not_reported_again(run):
+    """An allocation that failed is the error of its own call only."""
+    run("""
+p = P.structured(gf.GF_Q4, 9, 5)
+mesh = mesh_of(p)
+fake.fake_fail_at(0)
+try:
+    mesh_of(p)
+    assert False, "the upload was to fail"
+except gf.GpufemError:
+    pass
+ctx.symbolic(mesh)
+""")
