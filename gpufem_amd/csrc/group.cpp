@@ -115,32 +115,58 @@ int ensure_slice_groups(gf_ctx* ctx, gf_group* g) {
     }
     ptr[size_t(k) + 1] = int64_t(mesh.size());
   }
-  g->nsg = int64_t(mesh.size());
   const size_t ns = std::max<size_t>(mesh.size(), 1);
-  hipError_t e = hipMalloc(&g->d_sg_ptr, ptr.size() * 8);
-  if (e == hipSuccess) e = hipMalloc(&g->d_sg_s0, ns * 8);
-  if (e == hipSuccess) e = hipMalloc(&g->d_sg_s1, ns * 8);
-  if (e == hipSuccess) e = hipMalloc(&g->d_sg_mesh, ns * 4);
-  if (e == hipSuccess) e = hipMalloc(&g->part_sg, ns * 8);
+  // built aside and published as a whole: a failed allocation leaves the group
+  // as it was, and the next solve starts over
+  struct Arrays {
+    int64_t *ptr = nullptr, *s0 = nullptr, *s1 = nullptr, *sl_ptr = nullptr;
+    int32_t *mesh = nullptr, *sl_mesh = nullptr;
+    double *part = nullptr, *split = nullptr;
+    ~Arrays() {
+      dfree(ptr);
+      dfree(s0);
+      dfree(s1);
+      dfree(sl_ptr);
+      dfree(mesh);
+      dfree(sl_mesh);
+      dfree(part);
+      dfree(split);
+    }
+  } A;
+  hipError_t e = hipMalloc(&A.ptr, ptr.size() * 8);
+  if (e == hipSuccess) e = hipMalloc(&A.s0, ns * 8);
+  if (e == hipSuccess) e = hipMalloc(&A.s1, ns * 8);
+  if (e == hipSuccess) e = hipMalloc(&A.mesh, ns * 4);
+  if (e == hipSuccess) e = hipMalloc(&A.part, ns * 8);
   // the two-launch iteration's arrays
   const gf_ell* m = g->ell;
-  g->split = is_split_variant(iter_variant(group_variant(m), m->bslots, sizeof(double)));
-  if (g->split) {
+  const bool split = is_split_variant(iter_variant(group_variant(m), m->bslots, sizeof(double)));
+  if (split) {
     std::vector<int32_t> sm(static_cast<size_t>(m->bslices + 2 * g->nmesh), 0);
     for (int k = 0; k < g->nmesh; ++k)
       std::fill(sm.begin() + bs[size_t(k)], sm.begin() + bs[size_t(k) + 1], k);
     if (e == hipSuccess)
-      e = hipMalloc(&g->split_buf, size_t(m->n + m->bslices + 2 * g->nmesh) * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&g->d_sl_ptr, bs.size() * 8);
-    if (e == hipSuccess) e = hipMalloc(&g->d_sl_mesh, sm.size() * 4);
-    if (e == hipSuccess) e = hipMemcpy(g->d_sl_ptr, bs.data(), bs.size() * 8, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(g->d_sl_mesh, sm.data(), sm.size() * 4, hipMemcpyHostToDevice);
+      e = hipMalloc(&A.split, size_t(m->n + m->bslices + 2 * g->nmesh) * sizeof(double));
+    if (e == hipSuccess) e = hipMalloc(&A.sl_ptr, bs.size() * 8);
+    if (e == hipSuccess) e = hipMalloc(&A.sl_mesh, sm.size() * 4);
+    if (e == hipSuccess) e = hipMemcpy(A.sl_ptr, bs.data(), bs.size() * 8, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(A.sl_mesh, sm.data(), sm.size() * 4, hipMemcpyHostToDevice);
   }
-  if (e == hipSuccess) e = hipMemcpy(g->d_sg_ptr, ptr.data(), ptr.size() * 8, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(g->d_sg_s0, s0.data(), s0.size() * 8, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(g->d_sg_s1, s1.data(), s1.size() * 8, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(g->d_sg_mesh, mesh.data(), mesh.size() * 4, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(A.ptr, ptr.data(), ptr.size() * 8, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(A.s0, s0.data(), s0.size() * 8, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(A.s1, s1.data(), s1.size() * 8, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(A.mesh, mesh.data(), mesh.size() * 4, hipMemcpyHostToDevice);
   if (e != hipSuccess) return set_error(ctx, GF_ERR_NOMEM, std::string("gf_group_pcg: ") + hipGetErrorString(e));
+  g->nsg = int64_t(mesh.size());
+  g->split = split;
+  std::swap(g->d_sg_ptr, A.ptr);
+  std::swap(g->d_sg_s0, A.s0);
+  std::swap(g->d_sg_s1, A.s1);
+  std::swap(g->d_sg_mesh, A.mesh);
+  std::swap(g->part_sg, A.part);
+  std::swap(g->split_buf, A.split);
+  std::swap(g->d_sl_ptr, A.sl_ptr);
+  std::swap(g->d_sl_mesh, A.sl_mesh);
   return GF_OK;
 }
 

@@ -63,3 +63,36 @@ except gf.GpufemError:
     pass
 ctx.symbolic(mesh)
 """)
+
+
+def test_group_solve_after_a_failed_allocation(run):
+    """Whatever allocation of the first grouped solve fails, the next solve
+    builds everything it needs, and the group gives back all it took."""
+    run("""
+probs = [P.structured(gf.GF_Q4, 9, 5), P.structured(gf.GF_Q4, 20, 9)]
+fake.fake_stop(b"k_gs_product")     # the iteration itself does not run here
+
+def solve(fail):
+    before = fake.fake_live()
+    G = ctx.group(probs)
+    G.assemble()
+    G.apply_penalty()
+    start = fake.fake_mallocs()
+    if fail is not None:
+        fake.fake_fail_at(fail)
+        st = G.pcg(schedule=gf.GF_SCHED_KERNELS, raise_on_fail=False)[1]
+        fake.fake_fail_at(-1)
+        assert st.code in (-2, -3) and not launched("k_gs_product"), st.code
+    st = G.pcg(schedule=gf.GF_SCHED_KERNELS, raise_on_fail=False)[1]
+    assert launched("k_gs_product")
+    fake.fake_clear_log()
+    held, taken = fake.fake_live(), fake.fake_mallocs() - start
+    G.free()
+    assert fake.fake_live() == before
+    return held - before, taken
+
+held, taken = solve(None)
+assert taken > 20
+for k in range(taken):
+    assert solve(k)[0] == held, k
+""")
