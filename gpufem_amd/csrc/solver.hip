@@ -307,12 +307,13 @@ __device__ inline void phase_split_update(const PcgBuffers& B, int lb, int slot,
 }
 
 // Whether iteration `it` runs, from the residual sum every workgroup forms in
-// the same order; `lead` sets the state when it does not.
+// the same order.  `lead` records that sum, which is the one to report should
+// the iteration break down, and sets the state when the iteration does not run.
 __device__ inline bool split_goes_on(const PcgBuffers& B, int it, double rr, bool lead) {
   PcgState* st = B.st;
+  if (lead) st->rr = rr;
   if (!(rr <= st->rtol2 * st->bnorm2) && it < st->maxit) return true;
   if (lead) {
-    st->rr = rr;
     st->it = it;
     st->done = 1;
   }
@@ -371,10 +372,8 @@ __global__ __launch_bounds__(kNT) void k_split_check(PcgBuffers B, int parity) {
   __shared__ double sh[kNT / 64];
   const double rr = reduce_partials(B.part2 + B.nblocks, B.nblocks, sh);
   if (threadIdx.x == 0) {
-    PcgState* st = B.st;
-    st->rr = rr;
-    st->it = st->itv[parity];
-    (void)split_goes_on(B, st->it, rr, true);
+    B.st->it = B.st->itv[parity];
+    (void)split_goes_on(B, B.st->it, rr, true);
   }
 }
 

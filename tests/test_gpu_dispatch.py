@@ -90,6 +90,42 @@ def test_two_launch_iteration_breakdown(gpu_ctx):
         assert s.converged and s.iterations == 0 and not x.any()
 
 
+def weak_corner(t, nx, ny, nz, scale):
+    """A problem whose first three elements have `scale` (negative) times the
+    modulus: the matrix is indefinite, CG breaks down after a few iterations."""
+    p = P.structured(t, nx, ny, nz)
+    p.elem_E = np.full(p.conn.shape[0], p.E)
+    p.elem_E[:3] *= scale
+    p.f = np.random.default_rng(0).normal(size=p.ndof)
+    return p
+
+
+def weak_matrix(ctx, p):
+    mesh = ctx.upload_mesh(p.elem_type, p.ngauss, p.conn, p.coords, p.E, p.nu, elem_E=p.elem_E)
+    K = ctx.symbolic(mesh)
+    ctx.assemble(mesh, K)
+    return K
+
+
+@pytest.mark.parametrize("t,nx,ny,nz,its", [
+    (gf.GF_Q4, 80, 50, 0, 11), (gf.GF_Q8, 60, 25, 0, 8), (gf.GF_BRICK8, 12, 12, 12, 15)])
+def test_late_breakdown_reports_its_own_residual(gpu_ctx, t, nx, ny, nz, its):
+    """A breakdown between two looks of the host at the state, iteration `its`
+    in 64 bits on the CPU: every schedule of the two-launch iteration reports
+    that iteration and its residual, which is the thread-per-row solve's to the
+    rounding of a dozen iterations."""
+    p = weak_corner(t, nx, ny, nz, -0.1)
+    K, R = weak_matrix(gpu_ctx, p), weak_matrix(gpu_ctx, p)
+    gpu_ctx.tune(R, 0)
+    kw = dict(precond=gf.GF_PRECOND_NONE, raise_on_fail=False)
+    _, want = gpu_ctx.pcg(R, p.f, **kw)
+    assert want.code == gf.GF_ERR_BREAKDOWN and want.iterations == its
+    for sched in (gf.GF_SCHED_KERNELS, gf.GF_SCHED_GRAPH, gf.GF_SCHED_PERSISTENT):
+        _, s = gpu_ctx.pcg(K, p.f, schedule=sched, **kw)
+        assert s.code == gf.GF_ERR_BREAKDOWN and s.iterations == its
+        assert abs(s.relres - want.relres) <= 1e-9 * want.relres
+
+
 def test_group_two_launch_iteration(gpu_ctx):
     """A grouped solve whose matrix stays in the last-level cache, meshes of one
     element to several slices: each mesh as solved alone (its own stopping
