@@ -311,11 +311,12 @@ __global__ __launch_bounds__(kNT) void k_g_beta(GroupBuffers G) {
 // direction pass go (five launches before: 51.1 us an iteration on 64 Q4 plates
 // of 615 k rows in all, 33.4 now).
 // ---------------------------------------------------------------------------
-// whether mesh m runs iteration `it`; its lead thread records why not
+// whether mesh m runs iteration `it`; its lead thread records the residual sum
+// (the one to report should the iteration break down) and, if not, the end
 __device__ inline bool mesh_goes_on(const GroupBuffers& G, int m, int it, double rr, bool lead) {
+  if (lead) G.rr[m] = rr;
   if (!(rr <= G.st->rtol2 * G.bb[m]) && it < G.st->maxit) return true;
   if (lead) {
-    G.rr[m] = rr;
     G.it[m] = it;
     G.done[m] = 1;
   }
@@ -423,7 +424,6 @@ __global__ __launch_bounds__(kNT) void k_gs_check(GroupBuffers G) {
     reduce_partials2(G.part + t0, G.part + G.ntiles + t0, int(G.tile_ptr[m + 1] - t0), &rz, &rr,
                      sh);
     if (threadIdx.x == 0) {
-      G.rr[m] = rr;
       G.it[m] = G.it2[m];
       (void)mesh_goes_on(G, m, G.it2[m], rr, true);
     }

@@ -155,6 +155,28 @@ def test_group_two_launch_iteration(gpu_ctx):
         assert sc.code == gf.GF_ERR_NOCONV and ic.max() == 5
 
 
+def test_group_late_breakdown_reports_its_own_residual(gpu_ctx):
+    """Each mesh's breakdown (a few iterations in) is
+    reported with its own iteration, the group with the larger residual of
+    the two, to the rounding of a few iterations."""
+    probs = [weak_corner(gf.GF_Q8, 60, 25, 0, -0.5), weak_corner(gf.GF_Q8, 60, 25, 0, -0.5)]
+    probs[1].f = 2.0 * probs[1].f + 1.0
+    alone = []
+    for p in probs:
+        R = weak_matrix(gpu_ctx, p)
+        gpu_ctx.tune(R, 0)
+        alone.append(gpu_ctx.pcg(R, p.f, raise_on_fail=False)[1])
+        assert alone[-1].code == gf.GF_ERR_BREAKDOWN and 0 < alone[-1].iterations < 16
+    G = gpu_ctx.group(probs)
+    G.assemble()
+    for sched in (gf.GF_SCHED_KERNELS, gf.GF_SCHED_GRAPH):
+        _, s, its = G.pcg(schedule=sched, raise_on_fail=False)
+        assert s.code == gf.GF_ERR_BREAKDOWN
+        assert [int(i) for i in its] == [a.iterations for a in alone]
+        want = max(a.relres for a in alone)
+        assert abs(s.relres - want) <= 1e-9 * want
+
+
 @pytest.mark.parametrize("precision", [gf.GF_PREC_FP64, gf.GF_PREC_MIXED])
 @pytest.mark.parametrize("t,nx,ny,nz,nrhs", [
     (gf.GF_BRICK8, 1, 1, 1, 2), (gf.GF_BRICK8, 3, 3, 3, 9),                # 8 and 64 nodes
