@@ -473,8 +473,8 @@ int gf_ell_download(gf_ctx* ctx, const gf_ell* m, double* val, int32_t* col,
 // ---------------------------------------------------------------------------
 // node -> (element << 5 | local node) lists for the node-gather assembly,
 // ascending element id per node (its order of summation)
-static int ensure_n2e(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m) {
-  if (m->d_n2e) return GF_OK;
+static hipError_t ensure_n2e(const gf_mesh* mesh, gf_ell* m) {
+  if (m->d_n2e) return hipSuccess;
   const int64_t nn = mesh->nnodes, ne = mesh->nelem;
   const int nen = mesh->nen;
   std::vector<int64_t> ptr(size_t(nn) + 1, 0);
@@ -498,11 +498,18 @@ static int ensure_n2e(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m) {
   if (e != hipSuccess) {  // nothing half-built is left behind
     if (d_ptr) (void)hipFree(d_ptr);
     if (d_lst) (void)hipFree(d_lst);
-    return set_error(ctx, GF_ERR_HIP, std::string("node incidence: ") + hipGetErrorString(e));
+    return e;
   }
   m->d_n2e_ptr = d_ptr;
   m->d_n2e = d_lst;
-  return GF_OK;
+  return hipSuccess;
+}
+
+// the element tensors of variant 2
+static hipError_t ensure_tensors(const gf_mesh* mesh, gf_ell* m) {
+  if (m->d_etens) return hipSuccess;
+  const int64_t cnt = elem_tensor_doubles(mesh->type, mesh->nelem);
+  return hipMalloc(&m->d_etens, size_t(std::max<int64_t>(cnt, 1)) * sizeof(double));
 }
 
 // the node-gather kernel exists for the type and every node fits its slots
@@ -515,14 +522,8 @@ static bool gather_fits(const gf_mesh* mesh, const gf_ell* m) {
 static int assemble_with(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m, int variant, gf_timing* t) {
   const double h0 = now_ms();
   const bool node_rows = variant == 2 || variant == 3 || variant == 4;  // no scatter
-  if (node_rows) {
-    int s3 = ensure_n2e(ctx, mesh, m);
-    if (s3) return s3;
-  }
-  if (variant == 2 && !m->d_etens) {
-    const int64_t cnt = elem_tensor_doubles(mesh->type, mesh->nelem);
-    GF_HIP_CHECK(ctx, hipMalloc(&m->d_etens, size_t(std::max<int64_t>(cnt, 1)) * sizeof(double)));
-  }
+  if (node_rows) GF_HIP_CHECK(ctx, ensure_n2e(mesh, m));
+  if (variant == 2) GF_HIP_CHECK(ctx, ensure_tensors(mesh, m));
   if (variant == 4 && !m->d_egrad) {
     const int64_t cnt = gauss_geom_doubles(mesh->type, mesh->ngauss, mesh->nelem);
     GF_HIP_CHECK(ctx, hipMalloc(&m->d_egrad, size_t(std::max<int64_t>(cnt, 1)) * sizeof(double)));
@@ -608,11 +609,11 @@ static int assemble_with(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m, int varian
   return GF_OK;
 }
 
-// the element tensors (variant 2) must leave most of the device free
-static bool tensors_fit(const gf_mesh* mesh) {
+// the element tensors (variant 2) take at most this share of the free memory
+static bool tensors_fit(const gf_mesh* mesh, double share) {
   size_t free_b = 0, total_b = 0;
   const double need = double(elem_tensor_doubles(mesh->type, mesh->nelem)) * sizeof(double);
-  return hipMemGetInfo(&free_b, &total_b) == hipSuccess && need <= 0.5 * double(free_b);
+  return hipMemGetInfo(&free_b, &total_b) == hipSuccess && need <= share * double(free_b);
 }
 
 // The assembly kernel of a mesh too small to be worth timing (below 65536
@@ -627,9 +628,20 @@ static bool tensors_fit(const gf_mesh* mesh) {
 // points in the reference's order, and on slender plates (Q8 128x8, condition
 // number 1.5e8) the other rounding of the gather's entries moves the solution
 // by 1e-9, for 0.02 ms of a pass saved (Q4 64x32: 0.010 / 0.032 ms).
-static int small_mesh_variant(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m) {
-  if (mesh->dim != 3 || !gather_fits(mesh, m) || ensure_n2e(ctx, mesh, m) != GF_OK) return 0;
-  return mesh->type == GF_BRICK20 && tensors_fit(mesh) ? 2 : 3;
+// The scatter needs no memory of its own: where the gather's cannot be had it
+// is taken instead, and the tensors (28.8 KB an element, held with the matrix)
+// only from plenty: the solvers' workspaces are allocated after them.
+static int small_mesh_variant(const gf_mesh* mesh, gf_ell* m) {
+  if (mesh->dim != 3 || !gather_fits(mesh, m)) return 0;
+  int v = 0;
+  if (ensure_n2e(mesh, m) == hipSuccess) {
+    v = 3;
+    if (mesh->type == GF_BRICK20 && tensors_fit(mesh, 0.125) &&
+        ensure_tensors(mesh, m) == hipSuccess)
+      v = 2;
+  }
+  (void)hipGetLastError();  // a failed allocation is no error of the call
+  return v;
 }
 
 static int check_assembly_args(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m, const char* fn) {
@@ -679,7 +691,7 @@ int gf_assemble_tune(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m, int32_t force,
     for (int v : {0, 1, 3, 2}) {
       if ((v == 3 || v == 2) && !gather_fits(mesh, m)) continue;
       if (v == 2 && mesh->type != GF_BRICK20) continue;
-      if (v == 2 && !m->d_etens && !tensors_fit(mesh)) continue;
+      if (v == 2 && !m->d_etens && !tensors_fit(mesh, 0.5)) continue;
       gf_timing t1{}, t2{};
       if ((st = assemble_with(ctx, mesh, m, v, &t1)) || (st = assemble_with(ctx, mesh, m, v, &t2)))
         return st;
@@ -706,7 +718,7 @@ int gf_assemble(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m, gf_timing* t) {
   if (st) return st;
   if (m->asm_variant < 0) {
     // small meshes: not worth timing; large ones pick the fastest kernel once
-    if (m->nelem < 65536) m->asm_variant = small_mesh_variant(ctx, mesh, m);
+    if (m->nelem < 65536) m->asm_variant = small_mesh_variant(mesh, m);
     else if ((st = gf_assemble_tune(ctx, mesh, m, -1, nullptr, nullptr))) return st;
   }
   return assemble_with(ctx, mesh, m, m->asm_variant, t);

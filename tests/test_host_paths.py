@@ -96,3 +96,62 @@ assert taken > 20
 for k in range(taken):
     assert solve(k)[0] == held, k
 """)
+
+
+def test_first_assembly_of_a_small_mesh_needs_no_memory(run):
+    """The kernel of a small mesh is picked without timing; where its arrays
+    cannot be allocated the assembly runs all the same, then and later."""
+    run("""
+for p in (P.structured(gf.GF_BRICK8, 3, 2, 2), P.structured(gf.GF_BRICK20, 3, 2, 2)):
+    mesh = mesh_of(p)
+    k = 0
+    while True:
+        K = ctx.symbolic(mesh)
+        start = fake.fake_mallocs()
+        fake.fake_fail_at(k)
+        ctx.assemble(mesh, K)
+        fake.fake_fail_at(-1)
+        taken = fake.fake_mallocs() - start
+        ctx.assemble(mesh, K)
+        if k >= taken:
+            break
+        k += 1
+    assert k > 0
+""")
+
+
+def test_small_mesh_assembly_leaves_room_for_the_solve(run):
+    """With room for the scatter's assembly and a batched solve, and little
+    more, the untimed assembly leaves enough for that solve."""
+    run("""
+p = P.structured(gf.GF_BRICK20, 10, 10, 10)
+F = np.zeros((64, p.ndof))
+fake.fake_stop(b"k_mm_spmm_pq")     # the first kernel of an iteration
+mesh = mesh_of(p)
+
+def solve(force):
+    K = ctx.symbolic(mesh)
+    start = fake.fake_live_bytes()
+    if force is not None:
+        ctx.assemble_tune(mesh, K, force)
+    ctx.assemble(mesh, K)
+    fake.fake_clear_log()
+    x, st = ctx.pcg(K, F, precision=gf.GF_PREC_MIXED, schedule=gf.GF_SCHED_KERNELS,
+                    raise_on_fail=False)
+    reached = launched("k_mm_spmm_pq")
+    K.free()
+    return reached, start
+
+held = fake.fake_live_bytes()
+low, high = 1, 1 << 33              # the least memory in which it runs
+while high - low > 1 << 16:
+    mid = (low + high) // 2
+    fake.fake_memory(held + mid, 0)
+    try:
+        ok = solve(0)[0]
+    except gf.GpufemError:
+        ok = False
+    low, high = (low, mid) if ok else (mid, high)
+fake.fake_memory(held + int(1.02 * high), 0)
+assert solve(None)[0], "%.1f MB are too little" % (1.02e-6 * high)
+""")
