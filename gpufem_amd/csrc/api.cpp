@@ -34,6 +34,9 @@ int set_error(const gf_ctx* ctx, int code, const std::string& msg) {
 
 namespace {
 
+// elements; smaller meshes take their assembly kernel without timing
+constexpr int64_t kSmallMesh = 65536;
+
 double now_ms() {
   using namespace std::chrono;
   return duration<double, std::milli>(steady_clock::now().time_since_epoch()).count();
@@ -331,6 +334,8 @@ int gf_ell_symbolic_device(gf_ctx* ctx, const gf_mesh* mesh, gf_ell** out, gf_ti
     dfree(S.d_adj);
     dfree(S.d_slot);
     dfree(S.d_color_elems);
+    dfree(S.d_n2e_ptr);
+    dfree(S.d_n2e);
     m->d_slot = nullptr;
     m->d_color_elems = nullptr;
     ell_release(m.get());
@@ -365,6 +370,12 @@ int gf_ell_symbolic_device(gf_ctx* ctx, const gf_mesh* mesh, gf_ell** out, gf_ti
   (void)hipEventElapsedTime(&f, ctx->ev_start, ctx->ev_stop);
   dfree(S.d_adj_ptr);
   dfree(S.d_adj);
+  if (mesh->dim == 3 || mesh->nelem >= kSmallMesh) {  // the assembly tries the gather
+    std::swap(m->d_n2e_ptr, S.d_n2e_ptr);
+    std::swap(m->d_n2e, S.d_n2e);
+  }
+  dfree(S.d_n2e_ptr);
+  dfree(S.d_n2e);
   if (t) {
     t->ms_device = f;
     t->ms_host = now_ms() - h0;
@@ -472,37 +483,25 @@ int gf_ell_download(gf_ctx* ctx, const gf_ell* m, double* val, int32_t* col,
 
 // ---------------------------------------------------------------------------
 // node -> (element << 5 | local node) lists for the node-gather assembly,
-// ascending element id per node (its order of summation)
-static hipError_t ensure_n2e(const gf_mesh* mesh, gf_ell* m) {
-  if (m->d_n2e) return hipSuccess;
-  const int64_t nn = mesh->nnodes, ne = mesh->nelem;
-  const int nen = mesh->nen;
-  std::vector<int64_t> ptr(size_t(nn) + 1, 0);
-  for (int64_t i = 0; i < ne * nen; ++i) ptr[size_t(mesh->h_conn[size_t(i)])]++;
-  for (int64_t v = 0; v < nn; ++v) ptr[size_t(v) + 1] += ptr[size_t(v)];
-  std::vector<int32_t> lst(static_cast<size_t>(ptr[size_t(nn)]));
-  std::vector<int64_t> fill(ptr.begin(), ptr.end() - 1);
-  for (int64_t e = 0; e < ne; ++e)  // ascending e: each node's list comes out sorted
-    for (int a = 0; a < nen; ++a) {
-      const int64_t v = mesh->h_conn[size_t(e * nen + a)] - 1;
-      lst[size_t(fill[size_t(v)]++)] = int32_t((e << 5) | a);
-    }
-  int64_t* d_ptr = nullptr;
-  int32_t* d_lst = nullptr;
-  hipError_t e = hipMalloc(&d_ptr, ptr.size() * sizeof(int64_t));
-  if (e == hipSuccess) e = hipMalloc(&d_lst, std::max<size_t>(lst.size(), 1) * sizeof(int32_t));
+// ascending element id per node (its order of summation).  The device symbolic
+// phase leaves the elements of each node, which one launch orders: the first
+// assembly of Brick8 40^3 with everything it builds takes 0.18 ms, 0.84 with
+// lists made on the host and copied.
+static hipError_t ensure_n2e(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m) {
+  if (m->n2e_ordered) return hipSuccess;
+  hipError_t e = hipSuccess;
+  if (!m->d_n2e)
+    e = build_incidence(ctx->stream, mesh->d_conn, mesh->nelem, mesh->nen, mesh->nnodes,
+                        &m->d_n2e_ptr, &m->d_n2e);
   if (e == hipSuccess)
-    e = hipMemcpy(d_ptr, ptr.data(), ptr.size() * sizeof(int64_t), hipMemcpyHostToDevice);
-  if (e == hipSuccess)
-    e = hipMemcpy(d_lst, lst.data(), lst.size() * sizeof(int32_t), hipMemcpyHostToDevice);
-  if (e != hipSuccess) {  // nothing half-built is left behind
-    if (d_ptr) (void)hipFree(d_ptr);
-    if (d_lst) (void)hipFree(d_lst);
-    return e;
+    e = launch_incidence_order(ctx->stream, mesh->d_conn, mesh->nen, mesh->nnodes, m->d_n2e_ptr,
+                               m->d_n2e);
+  m->n2e_ordered = e == hipSuccess;
+  if (e != hipSuccess) {  // no half-ordered list is left behind
+    dfree(m->d_n2e_ptr);
+    dfree(m->d_n2e);
   }
-  m->d_n2e_ptr = d_ptr;
-  m->d_n2e = d_lst;
-  return hipSuccess;
+  return e;
 }
 
 // the element tensors of variant 2
@@ -522,7 +521,7 @@ static bool gather_fits(const gf_mesh* mesh, const gf_ell* m) {
 static int assemble_with(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m, int variant, gf_timing* t) {
   const double h0 = now_ms();
   const bool node_rows = variant == 2 || variant == 3 || variant == 4;  // no scatter
-  if (node_rows) GF_HIP_CHECK(ctx, ensure_n2e(mesh, m));
+  if (node_rows) GF_HIP_CHECK(ctx, ensure_n2e(ctx, mesh, m));
   if (variant == 2) GF_HIP_CHECK(ctx, ensure_tensors(mesh, m));
   if (variant == 4 && !m->d_egrad) {
     const int64_t cnt = gauss_geom_doubles(mesh->type, mesh->ngauss, mesh->nelem);
@@ -623,7 +622,9 @@ static bool tensors_fit(const gf_mesh* mesh, double share) {
 // takes a launch per color, clears the ELL values first and re-lays them out
 // for the solver afterwards.  Measured, a pass with the copy kept current:
 // Brick20 30x33x28 1.06 ms against 3.92 ms (24x24x24 0.55 / 1.99, 20x17x13
-// 0.20 / 0.73); Brick8 64x32x32 0.149 / 0.625.  The scatter stays for nodes
+// 0.20 / 0.73); Brick8 64x32x32 0.149 / 0.625.  The first assembly of a new
+// matrix, with the lists and tensors it builds: Brick8 10^3 0.07 / 0.11, 40^3
+// 0.18 / 0.58; Brick20 6^3 0.11 / 0.20, 30x33x28 1.05 / 3.57.  The scatter stays for nodes
 // with more neighbours than the gather holds, and in 2D: it sums the Gauss
 // points in the reference's order, and on slender plates (Q8 128x8, condition
 // number 1.5e8) the other rounding of the gather's entries moves the solution
@@ -631,10 +632,10 @@ static bool tensors_fit(const gf_mesh* mesh, double share) {
 // The scatter needs no memory of its own: where the gather's cannot be had it
 // is taken instead, and the tensors (28.8 KB an element, held with the matrix)
 // only from plenty: the solvers' workspaces are allocated after them.
-static int small_mesh_variant(const gf_mesh* mesh, gf_ell* m) {
+static int small_mesh_variant(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m) {
   if (mesh->dim != 3 || !gather_fits(mesh, m)) return 0;
   int v = 0;
-  if (ensure_n2e(mesh, m) == hipSuccess) {
+  if (ensure_n2e(ctx, mesh, m) == hipSuccess) {
     v = 3;
     if (mesh->type == GF_BRICK20 && tensors_fit(mesh, 0.125) &&
         ensure_tensors(mesh, m) == hipSuccess)
@@ -718,7 +719,7 @@ int gf_assemble(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m, gf_timing* t) {
   if (st) return st;
   if (m->asm_variant < 0) {
     // small meshes: not worth timing; large ones pick the fastest kernel once
-    if (m->nelem < 65536) m->asm_variant = small_mesh_variant(mesh, m);
+    if (m->nelem < kSmallMesh) m->asm_variant = small_mesh_variant(ctx, mesh, m);
     else if ((st = gf_assemble_tune(ctx, mesh, m, -1, nullptr, nullptr))) return st;
   }
   return assemble_with(ctx, mesh, m, m->asm_variant, t);

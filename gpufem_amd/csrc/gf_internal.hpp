@@ -103,9 +103,11 @@ struct gf_ell {
   int32_t* d_color_elems = nullptr;   // element ids grouped by color
   uint8_t* d_slot = nullptr;          // [nelem][nen][nen] node rank of b in adj(a)
   // node -> (element << 5 | local node), ascending element (node-gather
-  // assembly; lazily built)
+  // assembly; lazily built, or kept from the device symbolic phase as plain
+  // element ids in any order until n2e_ordered)
   int64_t* d_n2e_ptr = nullptr;
   int32_t* d_n2e = nullptr;
+  bool n2e_ordered = false;
   // J^-1 and w detJ E of every element at its Gauss points (assembly
   // variant 4; lazily built)
   double* d_egrad = nullptr;

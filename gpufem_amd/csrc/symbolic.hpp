@@ -31,6 +31,8 @@ struct SymbolicDevice {
   int32_t* d_adj = nullptr;          // sorted 0-based node ids per node
   uint8_t* d_slot = nullptr;         // [nelem][nen][nen]
   int32_t* d_color_elems = nullptr;  // element ids grouped by color, ascending
+  int64_t* d_n2e_ptr = nullptr;      // [nnodes+1]
+  int32_t* d_n2e = nullptr;          // incident elements per node, in any order
   std::vector<int32_t> elem_color;   // [nelem], 1-based (host copy)
   std::vector<int64_t> color_ptr;    // [ncolors+1]
   int64_t nadj = 0;
@@ -41,5 +43,13 @@ struct SymbolicDevice {
 
 int build_symbolic_device(hipStream_t s, const int32_t* d_conn, int64_t nelem, int nen,
                           int64_t nnodes, SymbolicDevice* out, std::string* err);
+
+// Incident elements per node (nnodes + 1 pointers; any order) of a checked
+// connectivity, and such lists put into the order the node gather sums in:
+// (element << 5 | local node), ascending.
+hipError_t build_incidence(hipStream_t s, const int32_t* d_conn, int64_t nelem, int nen,
+                           int64_t nnodes, int64_t** d_ptr, int32_t** d_n2e);
+hipError_t launch_incidence_order(hipStream_t s, const int32_t* d_conn, int nen, int64_t nnodes,
+                                  const int64_t* d_ptr, int32_t* d_n2e);
 
 }  // namespace gf

@@ -3,8 +3,9 @@
 // from the connectivity already resident there.
 //
 // Adjacency: node -> incident elements by counting, a scan and an atomic
-// fill (the order inside a node's list is arbitrary and nothing depends on
-// it); then one wavefront per node gathers its candidate nodes into LDS and
+// fill (the order inside a node's list is arbitrary and nothing here depends
+// on it; the node gather of the assembly orders the lists, launch_incidence_order);
+// then one wavefront per node gathers its candidate nodes into LDS and
 // writes the distinct ones in ascending order (rank = number of distinct
 // candidates below), which is the set the host phase sorts.
 //
@@ -70,6 +71,29 @@ __global__ void k_incidence_fill(const int32_t* __restrict__ conn, int64_t nelem
     const int64_t v = conn[t] - 1;
     const int32_t pos = atomicAdd(cursor + v, 1);
     n2e[ptr[v] + pos] = int32_t(t / nen);
+  }
+}
+
+// A node's incident elements become (element << 5 | local node), ascending; an
+// element that names the node several times stands there as often, its local
+// nodes ascending.  One thread per node (at most a few dozen entries).
+__global__ void k_incidence_order(const int32_t* __restrict__ conn, int nen,
+                                  const int64_t* __restrict__ ptr, int64_t nnodes, int32_t* n2e) {
+  for (int64_t v = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; v < nnodes;
+       v += int64_t(gridDim.x) * blockDim.x) {
+    const int64_t p0 = ptr[v], p1 = ptr[v + 1];
+    for (int64_t k = p0; k < p1; ++k) {
+      const int32_t e = n2e[k];
+      int before = 0;  // entries of this element already placed
+      for (int64_t j = p0; j < k; ++j) before += (n2e[j] >> 5) == e;
+      int a = 0;
+      for (; a < nen - 1; ++a)
+        if (conn[int64_t(e) * nen + a] == v + 1 && before-- == 0) break;
+      const int32_t key = (e << 5) | a;
+      int64_t j = k;
+      for (; j > p0 && n2e[j - 1] > key; --j) n2e[j] = n2e[j - 1];
+      n2e[j] = key;
+    }
   }
 }
 
@@ -334,7 +358,75 @@ struct DevScratch {
   }
 };
 
+// exclusive sums of n counts
+hipError_t exclusive_sum(hipStream_t s, DevScratch* tmp, const int32_t* in, int64_t* out,
+                         int64_t n) {
+  if (n <= 0) return hipSuccess;
+  const int64_t ntiles = (n + kScanItems - 1) / kScanItems;
+  int64_t* tile_sum = nullptr;
+  const hipError_t e = tmp->alloc(&tile_sum, size_t(ntiles));
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_scan_tile_sums, dim3(unsigned(ntiles)), dim3(kScanThreads), 0, s, in, n,
+                     tile_sum);
+  hipLaunchKernelGGL(k_scan_tile_offsets, dim3(1), dim3(kScanThreads), 0, s, tile_sum, ntiles);
+  hipLaunchKernelGGL(k_scan_apply, dim3(unsigned(ntiles)), dim3(kScanThreads), 0, s, in, n,
+                     tile_sum, out);
+  return hipGetLastError();
+}
+
+// Where each node's incident elements start (nnodes + 1 entries); cnt: nnodes + 1
+// counts of scratch, err: 1 after it where a node id is out of range.
+hipError_t incidence_ptr(hipStream_t s, DevScratch* tmp, const int32_t* conn, int64_t total,
+                         int64_t nnodes, int32_t* cnt, int32_t* err, int64_t* ptr) {
+  hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(nnodes + 1, 256, 16384)), dim3(256), 0, s, cnt,
+                     nnodes + 1, 0);
+  hipLaunchKernelGGL(k_incidence_count, dim3(grid_for(total, 256, 16384)), dim3(256), 0, s, conn,
+                     total, nnodes, cnt, err);
+  const hipError_t e = hipGetLastError();
+  // over nnodes + 1 entries, the last count 0: the total
+  return e != hipSuccess ? e : exclusive_sum(s, tmp, cnt, ptr, nnodes + 1);
+}
+
+// and those elements, in any order (cursor: nnodes counts of scratch)
+hipError_t incidence_fill(hipStream_t s, const int32_t* conn, int64_t nelem, int nen,
+                          int64_t nnodes, int32_t* cursor, const int64_t* ptr, int32_t* n2e) {
+  hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(nnodes, 256, 16384)), dim3(256), 0, s, cursor,
+                     nnodes, 0);
+  hipLaunchKernelGGL(k_incidence_fill, dim3(grid_for(nelem * nen, 256, 16384)), dim3(256), 0, s,
+                     conn, nelem, nen, ptr, cursor, n2e);
+  return hipGetLastError();
+}
+
 }  // namespace
+
+hipError_t build_incidence(hipStream_t s, const int32_t* conn, int64_t nelem, int nen,
+                           int64_t nnodes, int64_t** ptr, int32_t** n2e) {
+  DevScratch tmp;
+  int64_t* p = nullptr;
+  int32_t *l = nullptr, *cnt = nullptr, *err = nullptr;
+  hipError_t e = hipMalloc(&p, (size_t(nnodes) + 1) * sizeof(int64_t));
+  if (e == hipSuccess) e = hipMalloc(&l, size_t(std::max<int64_t>(nelem * nen, 1)) * sizeof(int32_t));
+  if (e == hipSuccess) e = tmp.alloc(&cnt, size_t(nnodes) + 1);
+  if (e == hipSuccess) e = tmp.alloc(&err, 1);
+  if (e == hipSuccess) e = incidence_ptr(s, &tmp, conn, nelem * nen, nnodes, cnt, err, p);
+  if (e == hipSuccess) e = incidence_fill(s, conn, nelem, nen, nnodes, cnt, p, l);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);  // before the scratch goes
+  if (e != hipSuccess) {
+    if (p) (void)hipFree(p);
+    if (l) (void)hipFree(l);
+    return e;
+  }
+  *ptr = p;
+  *n2e = l;
+  return hipSuccess;
+}
+
+hipError_t launch_incidence_order(hipStream_t s, const int32_t* conn, int nen, int64_t nnodes,
+                                  const int64_t* ptr, int32_t* n2e) {
+  hipLaunchKernelGGL(k_incidence_order, dim3(grid_for(nnodes, 256, 65536)), dim3(256), 0, s, conn,
+                     nen, ptr, nnodes, n2e);
+  return hipGetLastError();
+}
 
 int build_symbolic_device(hipStream_t s, const int32_t* d_conn, int64_t nelem, int nen,
                           int64_t nnodes, SymbolicDevice* out, std::string* err) {
@@ -347,36 +439,16 @@ int build_symbolic_device(hipStream_t s, const int32_t* d_conn, int64_t nelem, i
 #define TRY(expr)                              \
   if ((e = (expr)) != hipSuccess) return hip_fail(#expr)
   const int64_t total = nelem * nen;
-  int32_t *d_cnt = nullptr, *d_cursor = nullptr, *d_n2e = nullptr, *d_flags = nullptr;
-  int64_t* d_n2e_ptr = nullptr;
+  int32_t *d_cnt = nullptr, *d_cursor = nullptr, *d_flags = nullptr;
   TRY(tmp.alloc(&d_flags, 4));  // [0] error code, [1] max count, [2] pending
   TRY(tmp.alloc(&d_cnt, size_t(nnodes) + 1));
   TRY(tmp.alloc(&d_cursor, size_t(nnodes)));
-  TRY(tmp.alloc(&d_n2e_ptr, size_t(nnodes) + 1));
-  TRY(tmp.alloc(&d_n2e, size_t(total)));
+  TRY(hipMalloc(&out->d_n2e_ptr, (size_t(nnodes) + 1) * sizeof(int64_t)));
+  TRY(hipMalloc(&out->d_n2e, size_t(std::max<int64_t>(total, 1)) * sizeof(int32_t)));
+  const int64_t* d_n2e_ptr = out->d_n2e_ptr;
+  const int32_t* d_n2e = out->d_n2e;
   hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, d_flags, int64_t(4), 0);
-  hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(nnodes + 1, 256, 16384)), dim3(256), 0, s, d_cnt,
-                     nnodes + 1, 0);
-  hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(nnodes, 256, 16384)), dim3(256), 0, s, d_cursor,
-                     nnodes, 0);
-  hipLaunchKernelGGL(k_incidence_count, dim3(grid_for(total, 256, 16384)), dim3(256), 0, s,
-                     d_conn, total, nnodes, d_cnt, d_flags);
-  TRY(hipGetLastError());
-  // exclusive sums (over nnodes + 1 entries, the last count 0: the total)
-  auto exclusive_sum = [&](const int32_t* in, int64_t* outp, int64_t n) -> hipError_t {
-    if (n <= 0) return hipSuccess;
-    const int64_t ntiles = (n + kScanItems - 1) / kScanItems;
-    int64_t* tile_sum = nullptr;
-    hipError_t r = tmp.alloc(&tile_sum, size_t(ntiles));
-    if (r != hipSuccess) return r;
-    hipLaunchKernelGGL(k_scan_tile_sums, dim3(unsigned(ntiles)), dim3(kScanThreads), 0, s, in, n,
-                       tile_sum);
-    hipLaunchKernelGGL(k_scan_tile_offsets, dim3(1), dim3(kScanThreads), 0, s, tile_sum, ntiles);
-    hipLaunchKernelGGL(k_scan_apply, dim3(unsigned(ntiles)), dim3(kScanThreads), 0, s, in, n,
-                       tile_sum, outp);
-    return hipGetLastError();
-  };
-  TRY(exclusive_sum(d_cnt, d_n2e_ptr, nnodes + 1));
+  TRY(incidence_ptr(s, &tmp, d_conn, total, nnodes, d_cnt, d_flags, out->d_n2e_ptr));
   int32_t h_flags[4] = {0, 0, 0, 0};
   TRY(hipMemcpyAsync(h_flags, d_flags, sizeof(h_flags), hipMemcpyDeviceToHost, s));
   TRY(hipStreamSynchronize(s));
@@ -384,9 +456,7 @@ int build_symbolic_device(hipStream_t s, const int32_t* d_conn, int64_t nelem, i
     *err = "connectivity references a node outside 1.." + std::to_string(nnodes);
     return GF_ERR_ARG;
   }
-  hipLaunchKernelGGL(k_incidence_fill, dim3(grid_for(total, 256, 16384)), dim3(256), 0, s, d_conn,
-                     nelem, nen, d_n2e_ptr, d_cursor, d_n2e);
-  TRY(hipGetLastError());
+  TRY(incidence_fill(s, d_conn, nelem, nen, nnodes, d_cursor, d_n2e_ptr, out->d_n2e));
 
   // node adjacency
   const int gnodes = int(std::min<int64_t>(std::max<int64_t>(nnodes, 1), 65536));
@@ -395,7 +465,7 @@ int build_symbolic_device(hipStream_t s, const int32_t* d_conn, int64_t nelem, i
   TRY(hipGetLastError());
   hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, d_cnt + nnodes, int64_t(1), 0);
   TRY(hipMalloc(&out->d_adj_ptr, (size_t(nnodes) + 1) * sizeof(int64_t)));
-  TRY(exclusive_sum(d_cnt, out->d_adj_ptr, nnodes + 1));
+  TRY(exclusive_sum(s, &tmp, d_cnt, out->d_adj_ptr, nnodes + 1));
   int64_t nadj = 0;
   TRY(hipMemcpyAsync(&nadj, out->d_adj_ptr + nnodes, sizeof(int64_t), hipMemcpyDeviceToHost, s));
   TRY(hipMemcpyAsync(h_flags, d_flags, sizeof(h_flags), hipMemcpyDeviceToHost, s));
@@ -465,7 +535,7 @@ int build_symbolic_device(hipStream_t s, const int32_t* d_conn, int64_t nelem, i
     hipLaunchKernelGGL(k_color_tile_counts, dim3(gt), dim3(kColorThreads), 0, s, d_color, nelem,
                        ntiles, d_tcnt);
     TRY(hipGetLastError());
-    TRY(exclusive_sum(d_tcnt, d_toff, 64 * ntiles));
+    TRY(exclusive_sum(s, &tmp, d_tcnt, d_toff, 64 * ntiles));
     hipLaunchKernelGGL(k_color_tile_scatter, dim3(gt), dim3(kColorThreads), 0, s, d_color, nelem,
                        ntiles, d_toff, out->d_color_elems);
     TRY(hipGetLastError());

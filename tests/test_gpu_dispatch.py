@@ -266,3 +266,46 @@ def test_gather_adds_alike_and_turned_elements(gpu_ctx, t, nx, ny, nz, variant, 
     Ko, _ = O.assemble(g.dim, ng, conn, coords, 210000.0, 0.3, skip_zero=False)
     ov = Ko.export(Ko.max_rownnz())[0]
     assert np.abs(val - ov).max() <= 1e-12 * np.abs(ov).max()
+
+
+def collapsed(conn, coords):
+    """A corner edge of the box drawn together: the elements around it name
+    one node twice."""
+    X = coords
+    a = np.nonzero(np.all(X == X.min(0), axis=1))[0][0]
+    d = np.linalg.norm(X - X[a], axis=1)
+    b = np.nonzero((d > 0) & np.all(X[:, 1:] == X[a, 1:], axis=1))[0]
+    b = b[np.argmin(d[b])]
+    out = np.where(conn == b + 1, a + 1, conn)
+    return np.where(out > b + 1, out - 1, out), np.delete(coords, b, axis=0)
+
+
+@pytest.mark.parametrize("t,nx,ny,nz,variant,form", [
+    (gf.GF_BRICK8, 1, 1, 1, 3, ""), (gf.GF_BRICK8, 6, 5, 4, 3, "shuffled"),
+    (gf.GF_BRICK8, 4, 3, 3, 3, "collapsed"), (gf.GF_BRICK20, 3, 4, 2, 2, "shuffled"),
+    (gf.GF_Q8, 9, 7, 0, 3, "shuffled")])
+def test_gather_lists_made_on_the_device(gpu_ctx, t, nx, ny, nz, variant, form):
+    """The lists the node gather sums in order, after either symbolic phase
+    (the device one leaves unordered lists): the same bits, and the oracle's
+    values to 1e-12 of the largest."""
+    g = gf.Grid(t, nx, ny, nz)
+    conn, coords = g.fill()
+    conn = np.asarray(conn).reshape(g.nelem, -1)
+    if form == "collapsed":
+        conn, coords = collapsed(conn, coords)
+        assert any(len(set(c)) < conn.shape[1] for c in conn.tolist())
+    rng = np.random.default_rng(4)
+    conn = rng.permutation(conn) if form else conn
+    coords = coords + 0.03 * rng.uniform(-1, 1, coords.shape)
+    ng = 3 if t in (gf.GF_Q8, gf.GF_BRICK20) else 2
+    mesh = gpu_ctx.upload_mesh(t, ng, conn, coords, 210000.0, 0.3)
+    vals = []
+    for device in (False, True, True):
+        K = gpu_ctx.symbolic(mesh, device=device)
+        gpu_ctx.assemble_tune(mesh, K, variant)
+        gpu_ctx.assemble(mesh, K)
+        vals.append(gpu_ctx.download(K)[0])
+    assert np.array_equal(vals[0], vals[1]) and np.array_equal(vals[0], vals[2])
+    Ko, _ = O.assemble(g.dim, ng, conn, coords, 210000.0, 0.3, skip_zero=False)
+    ov = Ko.export(Ko.max_rownnz())[0]
+    assert np.abs(vals[0] - ov).max() <= 1e-12 * np.abs(ov).max()

@@ -155,3 +155,16 @@ while high - low > 1 << 16:
 fake.fake_memory(held + int(1.02 * high), 0)
 assert solve(None)[0], "%.1f MB are too little" % (1.02e-6 * high)
 """)
+
+
+def test_first_assembly_copies_no_lists(run):
+    """The node gather's lists are made on the device: the first assembly of a
+    mesh that is already there sends nothing to it."""
+    run("""
+for p in (P.structured(gf.GF_BRICK8, 9, 9, 9), P.structured(gf.GF_BRICK20, 4, 4, 4)):
+    mesh = mesh_of(p)
+    K = ctx.symbolic(mesh)
+    sent = fake.fake_h2d()
+    ctx.assemble(mesh, K)
+    assert launched("k_assemble_gather") and fake.fake_h2d() == sent
+""")
