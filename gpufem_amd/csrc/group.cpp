@@ -140,7 +140,7 @@ int ensure_slice_groups(gf_ctx* ctx, gf_group* g) {
   if (e == hipSuccess) e = hipMalloc(&A.part, ns * 8);
   // the two-launch iteration's arrays
   const gf_ell* m = g->ell;
-  const bool split = is_split_variant(iter_variant(group_variant(m), m->bslots, sizeof(double)));
+  const bool split = is_split_variant(iter_variant(group_variant(m), m->bslots, m->n));
   if (split) {
     std::vector<int32_t> sm(static_cast<size_t>(m->bslices + 2 * g->nmesh), 0);
     for (int k = 0; k < g->nmesh; ++k)

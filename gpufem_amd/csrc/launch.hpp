@@ -122,8 +122,20 @@ inline bool is_bsell_variant(int v) {
 // grid sweeps the slices (for_rows_split).
 enum IterVariant { kSplit2 = 11, kSplit3 = 12 };
 inline bool is_split_variant(int v) { return v == kSplit2 || v == kSplit3; }
-// what the last-level cache holds
-constexpr int64_t kCacheBytes = int64_t(256) << 20;
+// Where the split kernels stop: block values that stay in the last-level cache of
+// 256 MiB, and what an iteration moves, values, 16-bit columns and 96 bytes a row
+// (six vectors, read and written or read twice).  us an iteration, three launches /
+// two (two runs where they differ): around 328 MiB (344 MB) of the latter Q4 820x820
+// (336 MB) 69.0 / 67.0, 840x840 (352) 70.7 / 73.8, 960x960 (460) 89 / 109, Q8 560x285
+// (349) 79.1 / 77.9, 568x288 (358) 79.4 / 84.8; 3D matrices meet the line of the
+// values, 240 MiB (252 MB), first: Brick20 24^3 (244 MB) 62.7 / 55.5-58.4, Brick8
+// 50^3 (250) 67.3 / 63.8, Brick20 25x24x24 (254) 63.0 / 63.3-64.5, Brick8 51x51x50
+// (260) 68.4 / 66.0-70.0.
+constexpr int64_t kCacheBytes = int64_t(240) << 20;
+constexpr int64_t kCacheTraffic = int64_t(328) << 20;
+constexpr int64_t iteration_bytes(int64_t bslots, int d, int64_t n) {
+  return bslots * 64 * (d * d * 8 + 2) + 96 * n;
+}
 // node columns: coln[i + j n] = col[i + d j n] / d for j < width / d
 hipError_t launch_build_coln(hipStream_t s, int64_t n, int32_t width, int d, const int32_t* col,
                              int32_t* coln);
@@ -188,9 +200,9 @@ int spmv_blocks(int64_t n);
 // the slice-group variants, else `nblocks`
 int spmv_grid(int variant, const BsellView& bs, int nblocks);
 // the kernel that forms q = K p inside an iteration: the split kernels for the
-// slice-group variants while the block values (bslots block slots of
-// value_bytes each) stay in the last-level cache, else the variant itself
-int iter_variant(int variant, int64_t bslots, int64_t value_bytes);
+// slice-group variants while a matrix of n rows and bslots block slots stays in
+// the last-level cache, else the variant itself
+int iter_variant(int variant, int64_t bslots, int64_t n);
 // Whether the iterations of such a matrix run in one workgroup (k_single): its
 // vectors fit the LDS and registers of a CU, and its values are read there
 // sooner (about 120 GB/s past the held ones) than two launches take.  us an

@@ -115,7 +115,7 @@ extern "C" int gf_pcg_noalloc(gf_ctx* ctx, gf_ell* m, const double* b, double* x
   B.n = n;
   B.width = m->width;
   B.variant = variant;
-  B.iter_variant = iter_variant(variant, m->bslots, sizeof(double));
+  B.iter_variant = iter_variant(variant, m->bslots, m->n);
   B.single = single_fits(B.iter_variant, n, m->bslots, o.bs.nslices);
   B.val = o.val;
   B.col = o.col;

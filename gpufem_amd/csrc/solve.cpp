@@ -99,7 +99,7 @@ void set_variant(gf_ell* m, int variant) {
   if (P->variant == variant && P->nblocks > 0) return;
   drop_graphs(P);
   P->variant = variant;
-  const int iter = iter_variant(variant, m->bslots, sizeof(double));
+  const int iter = iter_variant(variant, m->bslots, m->n);
   P->persistent_ok = persistent_blocks(iter, P->num_cu) > 0;
   P->nblocks = pcg_grid(iter, m->n, P->num_cu);
 }
@@ -289,7 +289,7 @@ PcgBuffers make_buffers(gf_ell* m, const double* dinv) {
   B.n = m->n;
   B.width = m->width;
   B.variant = P->variant;
-  B.iter_variant = iter_variant(P->variant, m->bslots, sizeof(double));
+  B.iter_variant = iter_variant(P->variant, m->bslots, m->n);
   B.single = single_fits(B.iter_variant, m->n, m->bslots, o.bs.nslices);
   B.val = o.val;
   B.col = o.col;
@@ -316,7 +316,7 @@ int cached_variant(const gf_ell* m) {
   const int b = bsell_variant(m);
   if (b < 0 || !m->d_bperm) return -1;
   const int g = b == kBsell2 ? kBsell2G : kBsell3G;
-  return is_split_variant(iter_variant(g, m->bslots, sizeof(double))) ? g : -1;
+  return is_split_variant(iter_variant(g, m->bslots, m->n)) ? g : -1;
 }
 
 int tune_spmv(gf_ctx* ctx, gf_ell* m, int force, double* ms_out, int* chosen) {

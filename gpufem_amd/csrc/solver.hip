@@ -1040,10 +1040,12 @@ hipError_t launch_bsell_to_ell(hipStream_t s, const BsellView& bs, int d, int64_
   return hipGetLastError();
 }
 
-int iter_variant(int variant, int64_t bslots, int64_t value_bytes) {
+int iter_variant(int variant, int64_t bslots, int64_t n) {
   if (!is_bsell_group_variant(variant)) return variant;
   const int d = variant == kBsell2G ? 2 : 3;
-  if (bslots * 64 * d * d * value_bytes > kCacheBytes) return variant;
+  if (bslots * 64 * d * d * int64_t(sizeof(double)) > kCacheBytes ||
+      iteration_bytes(bslots, d, n) > kCacheTraffic)
+    return variant;
   return d == 2 ? kSplit2 : kSplit3;
 }
 

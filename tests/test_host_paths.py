@@ -168,3 +168,22 @@ for p in (P.structured(gf.GF_BRICK8, 9, 9, 9), P.structured(gf.GF_BRICK20, 4, 4,
     ctx.assemble(mesh, K)
     assert launched("k_assemble_gather") and fake.fake_h2d() == sent
 """)
+
+
+def test_two_launch_iteration_up_to_the_cache(run):
+    """The iteration a solve runs on both sides of the line between matrices
+    that stay in the last-level cache and those that do not."""
+    run("""
+fake.fake_stop(b"_update")          # the second launch of an iteration
+for t, nx, ny, two in ((gf.GF_Q4, 700, 700, True), (gf.GF_Q4, 840, 840, False),
+                       (gf.GF_Q8, 540, 275, True), (gf.GF_Q8, 576, 290, False),
+                       (gf.GF_BRICK8, 50, 50, True), (gf.GF_BRICK8, 51, 51, False)):
+    p = P.structured(t, nx, ny, 50 if t == gf.GF_BRICK8 else 0)
+    mesh = mesh_of(p)
+    K = ctx.symbolic(mesh)
+    ctx.assemble(mesh, K)
+    fake.fake_clear_log()
+    ctx.pcg(K, p.f, schedule=gf.GF_SCHED_KERNELS, raise_on_fail=False)
+    assert launched("k_split_product") == two, (nx, ny)
+    assert launched("k_spmv_pq") != two
+""")
