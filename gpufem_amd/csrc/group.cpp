@@ -99,6 +99,29 @@ int group_variant(const gf_ell* m) {
   return kThreadU8;
 }
 
+// Whether the group's iteration takes two launches (the block-sliced copy is
+// built).  Three of five launches go, so values up to the whole cache gain; the
+// bytes an iteration moves are bounded more tightly than the single system's
+// (kCacheTraffic), since every workgroup also adds the partials of its whole mesh,
+// and the mesh with the most tiles bounds that.  us an iteration, five launches / two: Q4 plates 64 of 80x40
+// 45.3 / 29.4, 2 of 600x500 (2,353 tiles each; 300 MB an iteration) 80.2 / 73.3, 3 of
+// 500x450 (1,766; 337 MB) 83.7 / 89.6, 4 of 450x400 (347 MB) 86.0 / 93.5; one plate
+// of 600x600 (2,822 tiles) 60.9 / 55.5, 700x700 (3,840) 70.3 / 74.4, 840x840 (5,526)
+// 94.8 / 139; one Q8 plate of 380x380 (3,397; 316 MB) 93.3 / 88.8, 400x390 (340 MB)
+// 100 / 104; 2 Brick8 cubes of 40^3 (303 MB) 80.3 / 71.0.
+constexpr int64_t kGroupBytes = int64_t(256) << 20, kGroupTraffic = int64_t(304) << 20;
+constexpr int64_t kGroupTiles = 3400;
+bool group_split(const gf_group* g) {
+  const gf_ell* m = g->ell;
+  if (!is_bsell_group_variant(group_variant(m)) ||
+      m->bslots * 64 * m->dim * m->dim * int64_t(sizeof(double)) > kGroupBytes ||
+      iteration_bytes(m->bslots, m->dim, m->n) > kGroupTraffic)
+    return false;
+  for (int k = 0; k < g->nmesh; ++k)
+    if (g->tile_ptr[size_t(k) + 1] - g->tile_ptr[size_t(k)] > kGroupTiles) return false;
+  return true;
+}
+
 // slice groups per mesh from the block-sliced structure (once)
 int ensure_slice_groups(gf_ctx* ctx, gf_group* g) {
   if (g->d_sg_ptr) return GF_OK;
@@ -140,7 +163,7 @@ int ensure_slice_groups(gf_ctx* ctx, gf_group* g) {
   if (e == hipSuccess) e = hipMalloc(&A.part, ns * 8);
   // the two-launch iteration's arrays
   const gf_ell* m = g->ell;
-  const bool split = is_split_variant(iter_variant(group_variant(m), m->bslots, m->n));
+  const bool split = group_split(g);
   if (split) {
     std::vector<int32_t> sm(static_cast<size_t>(m->bslices + 2 * g->nmesh), 0);
     for (int k = 0; k < g->nmesh; ++k)

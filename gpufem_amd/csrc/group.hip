@@ -306,9 +306,9 @@ __global__ __launch_bounds__(kNT) void k_g_beta(GroupBuffers G) {
 // ---------------------------------------------------------------------------
 // The two-launch iteration of a group whose matrix stays in the last-level
 // cache (the single system's, solver.hip, with the scalars of each mesh).  A
-// workgroup belongs to one mesh, so it adds that mesh's partials itself: a few
-// hundred at most, one load per thread.  The two reduction launches and the
-// direction pass go (five launches before: 51.1 us an iteration on 64 Q4 plates
+// workgroup belongs to one mesh, so it adds that mesh's partials itself: one load
+// per thread for a few hundred of them, and never more than group_split (group.cpp)
+// lets a mesh have.  The two reduction launches and the direction pass go (five launches before: 51.1 us an iteration on 64 Q4 plates
 // of 615 k rows in all, 33.4 now).
 // ---------------------------------------------------------------------------
 // whether mesh m runs iteration `it`; its lead thread records the residual sum

@@ -187,3 +187,20 @@ for t, nx, ny, two in ((gf.GF_Q4, 700, 700, True), (gf.GF_Q4, 840, 840, False),
     assert launched("k_split_product") == two, (nx, ny)
     assert launched("k_spmv_pq") != two
 """)
+
+
+def test_group_takes_two_launches_where_they_are_faster(run):
+    """Both borders of the grouped two-launch iteration: the bytes of an
+    iteration, and the tiles of the largest mesh."""
+    run("""
+fake.fake_stop(b"_update")
+for sizes, two in (([(600, 600)], True), ([(760, 760)], False), ([(600, 500)] * 2, True),
+                   ([(500, 450)] * 3, False), ([(760, 760), (5, 5)], False),
+                   ([(120, 60)] * 16, True)):
+    G = ctx.group([P.structured(gf.GF_Q4, *s) for s in sizes])
+    G.assemble()
+    fake.fake_clear_log()
+    G.pcg(schedule=gf.GF_SCHED_KERNELS, raise_on_fail=False)
+    assert launched("k_gs_product") == two, sizes
+    assert launched("k_g_spmv_pq_bs") != two
+""")
