@@ -280,10 +280,10 @@ struct PcgHostState {
   double rr, bnorm2;
 };
 hipError_t read_pcg_state(hipStream_t s, const PcgBuffers& B, PcgHostState* h);
-// nrep launches of the iteration's SpMV kernel with the state forced live; with
-// `direction` each is followed by the direction pass where that is separate
-hipError_t launch_spmv_pq_repeat(hipStream_t s, const PcgBuffers& B, int nrep,
-                                 bool direction = false);
+// nrep launches of the iteration's SpMV kernel with the state forced live
+hipError_t launch_spmv_pq_repeat(hipStream_t s, const PcgBuffers& B, int nrep);
+// a solve from zero that runs until it is left (b: B's right-hand side, filled here)
+hipError_t launch_probe_setup(hipStream_t s, const PcgBuffers& B, double* b);
 // true residual ||b - K x|| / ||b|| into *out (device), deterministic
 hipError_t launch_true_residual(hipStream_t s, const PcgBuffers& B, double* out_dev);
 // *out_dev = 1/2 x.Kx - b.x (B.q is overwritten with K x)

@@ -956,7 +956,14 @@ __global__ __launch_bounds__(kNT) void k_energy_finish(PcgBuffers B, int nb, dou
   if (threadIdx.x == 0) out[0] = 0.5 * xq - xb;
 }
 
-// a state in which products and direction passes run whatever the partials hold
+// a right-hand side no eigenvector of a stiffness matrix is like: 0.5 to 1.5, scattered
+__global__ void k_probe_rhs(int64_t n, double* b) {
+  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+       i += int64_t(gridDim.x) * blockDim.x)
+    b[i] = 0.5 + double((uint32_t(i) * 2654435761u) >> 8) * 0x1p-24;
+}
+
+// a state in which products run whatever the partials hold
 __global__ void k_state_live(PcgState* st) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     st->done = 0;
@@ -1281,17 +1288,17 @@ hipError_t read_pcg_state(hipStream_t s, const PcgBuffers& B, PcgHostState* h) {
   return hipSuccess;
 }
 
-hipError_t launch_spmv_pq_repeat(hipStream_t s, const PcgBuffers& B, int nrep, bool direction) {
+hipError_t launch_spmv_pq_repeat(hipStream_t s, const PcgBuffers& B, int nrep) {
   hipLaunchKernelGGL(k_state_live, dim3(1), dim3(64), 0, s, B.st);
   hipError_t e = hipGetLastError();
-  for (int i = 0; i < nrep && e == hipSuccess; ++i) {
-    e = launch_product(s, B, 0);
-    if (e == hipSuccess && direction && !is_split_variant(B.iter_variant)) {
-      hipLaunchKernelGGL(k_direction, dim3(B.nblocks), dim3(kNT), 0, s, B, 0);
-      e = hipGetLastError();
-    }
-  }
+  for (int i = 0; i < nrep && e == hipSuccess; ++i) e = launch_product(s, B, 0);
   return e;
+}
+
+hipError_t launch_probe_setup(hipStream_t s, const PcgBuffers& B, double* b) {
+  hipLaunchKernelGGL(k_probe_rhs, dim3(grid_for(B.n, kNT, 8192)), dim3(kNT), 0, s, B.n, b);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess ? e : launch_pcg_setup(s, B, 0, 0.0, INT32_MAX);
 }
 
 hipError_t launch_energy(hipStream_t s, const PcgBuffers& B, double* out_dev) {

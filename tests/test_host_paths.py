@@ -204,3 +204,22 @@ for sizes, two in (([(600, 600)], True), ([(760, 760)], False), ([(600, 500)] * 
     assert launched("k_gs_product") == two, sizes
     assert launched("k_g_spmv_pq_bs") != two
 """)
+
+
+def test_tuner_reports_products_and_compares_iterations(run):
+    """ms_per_variant is the product alone; a variant whose product is the
+    fastest is not taken when its iteration is not."""
+    run("""
+p = P.structured(gf.GF_Q8, 60, 25)
+mesh = mesh_of(p)
+for update, want in ((20.0, False), (2.0, True)):
+    for name, us in ((b"k_spmv_pq", 6.0), (b"k_direction", 3.0), (b"k_update", 1.0),
+                     (b"k_split_product", 5.0), (b"k_split_update", update)):
+        fake.fake_cost(name, us)
+    K = ctx.symbolic(mesh)
+    ctx.assemble(mesh, K)
+    chosen, ms = ctx.tune(K)
+    assert (chosen == 9) == want, (chosen, ms)
+    # 16 products and one launch that readies the state
+    assert abs(ms[0] - 6.0e-3) < 1e-4 and abs(ms[9] - 5.0e-3) < 1e-4, ms
+""")
