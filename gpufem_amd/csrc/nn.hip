@@ -654,9 +654,10 @@ hipError_t launch_conv(hipStream_t s, const ConvArgs& a) {
 }
 
 size_t conv_fragments(int cin, int cout) {
-  // either direction's: the larger of the two slab counts, rounded to pairs
-  return size_t((27 * (cin >> 4) + 1) / 2) * (cout >> 4) * 512 +
-         size_t((27 * (cout >> 4) + 1) / 2) * (cin >> 4) * 512;
+  // either direction's: slabs are paired along the channels it sums over
+  const size_t fwd = size_t((27 * (cin >> 4) + 1) / 2) * (cout >> 4);
+  const size_t bwd = size_t((27 * (cout >> 4) + 1) / 2) * (cin >> 4);
+  return (fwd > bwd ? fwd : bwd) * 512;
 }
 
 namespace {

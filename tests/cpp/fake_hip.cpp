@@ -19,7 +19,7 @@ namespace {
 struct Fake {
   std::unordered_map<void*, size_t> mem;
   size_t live_bytes = 0, total_bytes = size_t(8) << 30, largest = ~size_t(0);
-  int64_t mallocs = 0, fail_at = -1, h2d = 0;
+  int64_t mallocs = 0, fail_at = -1, h2d = 0, last_bytes = 0;
   hipError_t last = hipSuccess;
   double clock_ms = 0.0;
   std::map<std::string, double> cost_us;  // by part of the name; else 1
@@ -83,6 +83,7 @@ int64_t fake_live() { return int64_t(F().mem.size()); }
 int64_t fake_live_bytes() { return int64_t(F().live_bytes); }
 int64_t fake_mallocs() { return F().mallocs; }
 int64_t fake_h2d() { return F().h2d; }
+int64_t fake_last_bytes() { return F().last_bytes; }  // of the last allocation asked for
 const char* fake_log() { return F().log.c_str(); }
 void fake_clear_log() { F().log.clear(); }
 
@@ -119,6 +120,7 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int
 hipError_t hipMalloc(void** p, size_t bytes) {
   *p = nullptr;
   const int64_t k = F().mallocs++;
+  F().last_bytes = int64_t(bytes);
   if (k == F().fail_at || bytes > F().largest || F().live_bytes + bytes > F().total_bytes)
     return err(hipErrorOutOfMemory);
   *p = std::calloc(bytes > 0 ? bytes : 1, 1);

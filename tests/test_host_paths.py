@@ -17,7 +17,7 @@ fake.fake_fail_at.argtypes = [C.c_int64]
 fake.fake_memory.argtypes = [C.c_int64, C.c_int64]
 fake.fake_cost.argtypes = [C.c_char_p, C.c_double]
 fake.fake_log.restype = C.c_char_p
-for f in ("live", "live_bytes", "mallocs", "h2d"):
+for f in ("live", "live_bytes", "mallocs", "h2d", "last_bytes"):
     getattr(fake, "fake_" + f).restype = C.c_int64
 sys.path.insert(0, %r)
 import numpy as np
@@ -222,4 +222,18 @@ for update, want in ((20.0, False), (2.0, True)):
     assert (chosen == 9) == want, (chosen, ms)
     # 16 products and one launch that readies the state
     assert abs(ms[0] - 6.0e-3) < 1e-4 and abs(ms[9] - 5.0e-3) < 1e-4, ms
+""")
+
+
+def test_convolution_fragments_take_one_direction(run):
+    """A weight buffer holds the fragments of one direction: pairs of
+    16-channel slabs of the 27 taps, 512 values each per output tile."""
+    run("""
+dims = np.array([9, 9, 9], dtype=np.int32)
+buf = gf.DevBuf(ctx, 9 ** 3 * 256 * 4)
+for cin, cout in ((16, 16), (16, 64), (192, 64), (128, 16)):
+    ctx._check(ctx.lib.gf_nn_conv3d(ctx.handle, buf.ptr, 1, gf._ptr(dims), cin, buf.ptr, None, cout,
+                                    1, 0, 0, 0.0, gf._ptr(dims), buf.ptr, None, 0))
+    one = [-(-27 * (a // 16) // 2) * (b // 16) * 512 for a, b in ((cin, cout), (cout, cin))]
+    assert fake.fake_last_bytes() == 2 * max(one), (cin, cout)
 """)
