@@ -43,10 +43,24 @@ def assembled(ctx, t, nx, ny, nz):
     return p, K
 
 
-@pytest.mark.parametrize("t,nx,ny,nz", [
-    (gf.GF_Q4, 1, 1, 0), (gf.GF_Q4, 7, 7, 0), (gf.GF_Q4, 20, 2, 0),      # 4, 64 and 63 nodes
-    (gf.GF_Q8, 33, 9, 0), (gf.GF_BRICK8, 1, 1, 1), (gf.GF_BRICK8, 15, 7, 7),
-    (gf.GF_BRICK20, 5, 4, 3), (gf.GF_Q4, 520, 519, 0)])                  # the last: two sweeps
+# what a solve whose caller chose no variant runs, by size: the iterations of a
+# small system in one workgroup, two launches an iteration, or three where the
+# matrix does not stay in the last-level cache (test_host_paths.py checks which)
+ONE_WORKGROUP = [
+    (gf.GF_Q4, 1, 1, 0), (gf.GF_Q4, 7, 7, 0), (gf.GF_Q4, 15, 7, 0),      # 1, 1 and 2 slices
+    (gf.GF_Q4, 20, 2, 0), (gf.GF_Q4, 47, 38, 0), (gf.GF_Q4, 63, 41, 0),
+    (gf.GF_Q4, 63, 42, 0),                                               # 0.744 of 0.750 MB
+    (gf.GF_Q8, 21, 13, 0), (gf.GF_Q8, 33, 9, 0), (gf.GF_BRICK8, 1, 1, 1), (gf.GF_BRICK8, 7, 7, 7),
+    (gf.GF_BRICK20, 2, 1, 1), (gf.GF_BRICK20, 4, 4, 3)]                  # 1.17 of 1.25 MB
+TWO_LAUNCHES = [
+    (gf.GF_Q4, 63, 43, 0),                                               # the first past it
+    (gf.GF_Q4, 80, 50, 0), (gf.GF_Q8, 40, 30, 0), (gf.GF_Q8, 60, 25, 0),
+    (gf.GF_BRICK8, 15, 7, 7), (gf.GF_BRICK8, 12, 12, 12), (gf.GF_BRICK20, 5, 4, 3),
+    (gf.GF_Q4, 520, 519, 0)]                                             # two sweeps
+THREE_LAUNCHES = [(gf.GF_Q4, 850, 850, 0), (gf.GF_BRICK8, 52, 51, 51)]
+
+
+@pytest.mark.parametrize("t,nx,ny,nz", TWO_LAUNCHES)
 def test_two_launch_iteration(gpu_ctx, t, nx, ny, nz):
     """A solve whose caller chose no variant takes the split kernels; its
     answer is the thread-per-row solve's at the same tolerance, preconditioned
@@ -74,20 +88,46 @@ def test_two_launch_iteration(gpu_ctx, t, nx, ny, nz):
                 assert ss.iterations == s.iterations and np.array_equal(xs, x)
 
 
-def test_two_launch_iteration_breakdown(gpu_ctx):
+@pytest.mark.parametrize("t,nx,ny,nz", [(gf.GF_Q4, 9, 5, 0),                # one workgroup
+                                        (gf.GF_Q4, 80, 50, 0), (gf.GF_BRICK8, 12, 12, 12)])
+def test_breakdown_at_the_start(gpu_ctx, t, nx, ny, nz):
     """A negative definite matrix breaks down at the first iteration and zero
     right-hand sides stop at none, on every schedule."""
-    g = gf.Grid(gf.GF_Q4, 9, 5)
+    g = gf.Grid(t, nx, ny, nz)
     conn, coords = g.fill()
-    mesh = gpu_ctx.upload_mesh(gf.GF_Q4, 2, conn, coords, -1.0, 0.3)
+    mesh = gpu_ctx.upload_mesh(t, 2, conn, coords, -1.0, 0.3)
     K = gpu_ctx.symbolic(mesh)
     gpu_ctx.assemble(mesh, K)
     f = np.random.default_rng(0).normal(size=g.ndof)
     for sched in (gf.GF_SCHED_KERNELS, gf.GF_SCHED_GRAPH, gf.GF_SCHED_PERSISTENT):
         x, s = gpu_ctx.pcg(K, f, schedule=sched, precond=gf.GF_PRECOND_NONE, raise_on_fail=False)
         assert s.code == gf.GF_ERR_BREAKDOWN and s.iterations == 0
+        assert s.relres == 1.0
         x, s = gpu_ctx.pcg(K, 0.0 * f, schedule=sched)
         assert s.converged and s.iterations == 0 and not x.any()
+
+
+@pytest.mark.parametrize("t,nx,ny,nz", THREE_LAUNCHES)
+def test_three_launches_past_the_cache(gpu_ctx, t, nx, ny, nz):
+    """The slice-group variant of a matrix that does not stay in the last-level
+    cache: its schedules agree bitwise, and after 20 iterations with the
+    thread-per-row variant to rounding (their products are the same bits, the
+    dot products' orders differ)."""
+    p = P.structured(t, nx, ny, nz)
+    mesh = gpu_ctx.upload_mesh(p.elem_type, p.ngauss, p.conn, p.coords, p.E, p.nu)
+    K = gpu_ctx.symbolic(mesh, device=True)
+    gpu_ctx.assemble(mesh, K)
+    gpu_ctx.apply_penalty(K, p.fixed_dofs)
+    kw = dict(rtol=0.0, maxit=20, verify=0, raise_on_fail=False)
+    gpu_ctx.tune(K, 9 if t == gf.GF_Q4 else 10)
+    x, s = gpu_ctx.pcg(K, p.f, schedule=gf.GF_SCHED_KERNELS, **kw)
+    assert s.iterations == 20
+    for sched in (gf.GF_SCHED_GRAPH, gf.GF_SCHED_PERSISTENT):
+        y, s2 = gpu_ctx.pcg(K, p.f, schedule=sched, **kw)
+        assert s2.iterations == 20 and np.array_equal(x, y) and s2.relres == s.relres
+    gpu_ctx.tune(K, 0)
+    y, s2 = gpu_ctx.pcg(K, p.f, **kw)
+    assert np.linalg.norm(x - y) <= 1e-9 * np.linalg.norm(y)
 
 
 def weak_corner(t, nx, ny, nz, scale):
@@ -199,11 +239,7 @@ def test_batched_rows_in_shares(gpu_ctx, t, nx, ny, nz, nrhs, precision):
     assert np.array_equal(X, Y) and s2.iterations == st.iterations
 
 
-@pytest.mark.parametrize("t,nx,ny,nz", [
-    (gf.GF_Q4, 1, 1, 0), (gf.GF_Q4, 7, 7, 0), (gf.GF_Q4, 15, 7, 0),      # 1, 1 and 2 slices
-    (gf.GF_Q4, 47, 38, 0), (gf.GF_Q4, 63, 41, 0), (gf.GF_Q4, 63, 42, 0),  # 42 slices is the last
-    (gf.GF_Q8, 21, 13, 0), (gf.GF_BRICK8, 1, 1, 1), (gf.GF_BRICK8, 7, 7, 7),
-    (gf.GF_BRICK20, 2, 1, 1), (gf.GF_BRICK20, 4, 4, 3)])
+@pytest.mark.parametrize("t,nx,ny,nz", ONE_WORKGROUP)
 @pytest.mark.parametrize("sched", [gf.GF_SCHED_KERNELS, gf.GF_SCHED_PERSISTENT])
 def test_small_system_in_one_workgroup(gpu_ctx, t, nx, ny, nz, sched):
     """Systems at the edges of the single workgroup's range: the residual
@@ -228,6 +264,23 @@ def test_small_system_in_one_workgroup(gpu_ctx, t, nx, ny, nz, sched):
     assert s5.iterations == min(3, st.iterations)
     z, s6 = gpu_ctx.pcg(K, np.zeros_like(f), schedule=sched)
     assert s6.iterations == 0 and not z.any()
+
+
+@pytest.mark.parametrize("nx", [1535, 1567])   # 48 slices, the most of one workgroup, and 49
+@pytest.mark.parametrize("sched", [gf.GF_SCHED_KERNELS, gf.GF_SCHED_PERSISTENT])
+def test_strip_at_the_slice_limit(gpu_ctx, nx, sched):
+    """A strip one element wide, with every slice of the single workgroup in
+    use and with one more: too ill-conditioned (1e13) to converge, so the
+    iterates of five iterations are compared with the thread-per-row solve."""
+    p, K = assembled(gpu_ctx, gf.GF_Q4, nx, 1, 0)
+    _, R = assembled(gpu_ctx, gf.GF_Q4, nx, 1, 0)
+    gpu_ctx.tune(R, 0)
+    f = np.random.default_rng(1).normal(size=p.ndof)
+    kw = dict(rtol=0.0, maxit=5, verify=0, raise_on_fail=False)
+    x, s = gpu_ctx.pcg(K, f, schedule=sched, **kw)
+    y, s2 = gpu_ctx.pcg(R, f, **kw)
+    assert s.iterations == 5 and s2.iterations == 5
+    assert np.linalg.norm(x - y) <= 1e-9 * np.linalg.norm(y)
 
 
 def turned(conn, coords):

@@ -396,11 +396,13 @@ def test_block_sliced_copy_tracks_new_values(gpu_ctx):
 
 
 @pytest.mark.parametrize("et,dims,variant", [(gf.GF_Q4, (64, 32), v) for v in (0, 2, 3, 4, 5, 7, 9)]
-                         + [(gf.GF_BRICK8, (9, 8, 7), v) for v in (6, 8, 10)])
+                         + [(gf.GF_BRICK8, (9, 8, 7), v) for v in (6, 8, 10)]
+                         + [(gf.GF_Q4, (80, 50), 9), (gf.GF_BRICK8, (24, 24, 24), 10)])
 def test_persistent_matches_kernel_schedule(gpu_ctx, et, dims, variant):
     """The persistent kernel plays the SpMV kernel's logical workgroups in
-    turn (more of them than co-resident ones for variants 9/10), so both
-    schedules reduce the same partials in the same order."""
+    turn (on the last two systems more of them than its grid has), so both
+    schedules reduce the same partials in the same order.  Variants 9/10 run the
+    two smaller systems in one workgroup under either schedule."""
     p, K = assembled(gpu_ctx, et, *dims)
     gpu_ctx.tune(K, variant)
     x1, s1 = gpu_ctx.pcg(K, p.f, schedule=gf.GF_SCHED_KERNELS)

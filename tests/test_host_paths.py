@@ -237,3 +237,36 @@ for cin, cout in ((16, 16), (16, 64), (192, 64), (128, 16)):
     one = [-(-27 * (a // 16) // 2) * (b // 16) * 512 for a, b in ((cin, cout), (cout, cin))]
     assert fake.fake_last_bytes() == 2 * max(one), (cin, cout)
 """)
+
+
+def test_gpu_tests_run_the_iterations_they_name(run):
+    """The sizes the GPU tests use for each kind of iteration lead to it, under
+    the kernel and the persistent schedule."""
+    run("""
+import os
+sys.path.insert(0, os.path.join(%r, "tests"))
+import test_gpu_dispatch as T
+
+def names(K, p, sched, stop):
+    fake.fake_stop(stop)
+    fake.fake_clear_log()
+    ctx.pcg(K, p.f, schedule=sched, raise_on_fail=False)
+    fake.fake_stop(b"")
+    return {n for n in ("k_single", "k_split_product", "k_spmv_pq", "k_split_persistent",
+                        "k_pcg_persistent") if launched(n)}
+
+for cases, kernel, stop, persistent in (
+        (T.ONE_WORKGROUP + [(gf.GF_Q4, 1535, 1, 0)], "k_single", b"k_single", "k_single"),
+        (T.TWO_LAUNCHES + [(gf.GF_Q4, 1567, 1, 0), (gf.GF_BRICK8, 24, 24, 24)],
+         "k_split_product", b"_update", "k_split_persistent"),
+        (T.THREE_LAUNCHES, "k_spmv_pq", b"_update", "k_pcg_persistent")):
+    for t, nx, ny, nz in cases:
+        p = P.structured(t, nx, ny, nz)
+        mesh = mesh_of(p)
+        K = ctx.symbolic(mesh)
+        ctx.assemble(mesh, K)
+        if kernel == "k_spmv_pq":
+            ctx.tune(K, 9 if nz == 0 else 10)
+        assert names(K, p, gf.GF_SCHED_KERNELS, stop) == {kernel}, (nx, ny, nz)
+        assert names(K, p, gf.GF_SCHED_PERSISTENT, persistent.encode()) == {persistent}, (nx, ny, nz)
+""" % ROOT)
