@@ -311,12 +311,11 @@ __global__ __launch_bounds__(kNT) void k_g_beta(GroupBuffers G) {
 // lets a mesh have.  The two reduction launches and the direction pass go (five launches before: 51.1 us an iteration on 64 Q4 plates
 // of 615 k rows in all, 33.4 now).
 // ---------------------------------------------------------------------------
-// whether mesh m runs iteration `it`; its lead thread records the residual sum
-// (the one to report should the iteration break down) and, if not, the end
+// whether mesh m runs iteration `it`; its lead thread records why not
 __device__ inline bool mesh_goes_on(const GroupBuffers& G, int m, int it, double rr, bool lead) {
-  if (lead) G.rr[m] = rr;
   if (!(rr <= G.st->rtol2 * G.bb[m]) && it < G.st->maxit) return true;
   if (lead) {
+    G.rr[m] = rr;
     G.it[m] = it;
     G.done[m] = 1;
   }
@@ -382,7 +381,13 @@ __global__ __launch_bounds__(kNT) void k_gs_update(GroupBuffers G, int parity) {
   if (done) return;
   const bool lead = threadIdx.x == 0 && t == G.tile_ptr[m];
   if (!(pq > 0.0)) {
+    // every workgroup of the mesh leaves here: its partials of r.r are still
+    // those of this iteration
+    if (t != G.tile_ptr[m]) return;
+    const double rr =
+        reduce_partials(G.part + G.ntiles + t, int(G.tile_ptr[m + 1] - t), sh);
     if (lead) {
+      G.rr[m] = rr;
       G.it[m] = it;
       G.status[m] = GF_ERR_BREAKDOWN;
       G.done[m] = 1;
@@ -424,6 +429,7 @@ __global__ __launch_bounds__(kNT) void k_gs_check(GroupBuffers G) {
     reduce_partials2(G.part + t0, G.part + G.ntiles + t0, int(G.tile_ptr[m + 1] - t0), &rz, &rr,
                      sh);
     if (threadIdx.x == 0) {
+      G.rr[m] = rr;
       G.it[m] = G.it2[m];
       (void)mesh_goes_on(G, m, G.it2[m], rr, true);
     }

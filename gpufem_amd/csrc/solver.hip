@@ -307,20 +307,24 @@ __device__ inline void phase_split_update(const PcgBuffers& B, int lb, int slot,
 }
 
 // Whether iteration `it` runs, from the residual sum every workgroup forms in
-// the same order.  `lead` records that sum, which is the one to report should
-// the iteration break down, and sets the state when the iteration does not run.
+// the same order; `lead` sets the state when it does not.
 __device__ inline bool split_goes_on(const PcgBuffers& B, int it, double rr, bool lead) {
   PcgState* st = B.st;
-  if (lead) st->rr = rr;
   if (!(rr <= st->rtol2 * st->bnorm2) && it < st->maxit) return true;
   if (lead) {
+    st->rr = rr;
     st->it = it;
     st->done = 1;
   }
   return false;
 }
-__device__ inline void split_breakdown(const PcgBuffers& B, int it, bool lead) {
-  if (!lead) return;
+// The iteration that breaks down reports its own residual: nothing has written
+// the partials of r.r since (every workgroup finds the same p.q and leaves).
+__device__ inline void split_breakdown(const PcgBuffers& B, int it, double* sh) {
+  if (blockIdx.x != 0) return;
+  const double rr = reduce_partials(B.part2 + B.nblocks, B.nblocks, sh);
+  if (threadIdx.x != 0) return;
+  B.st->rr = rr;
   B.st->it = it;
   B.st->status = GF_ERR_BREAKDOWN;
   B.st->done = 1;
@@ -360,7 +364,7 @@ __global__ __launch_bounds__(kNT) void k_split_update(PcgBuffers B, int parity) 
   const double rho = st->rho[parity], beta = split_beta(it, rho, st->rho[parity ^ 1]);
   const double pq = reduce_partials(B.part1, B.spmv_grid, sh);
   if (done) return;
-  if (!(pq > 0.0)) return split_breakdown(B, it, lead);
+  if (!(pq > 0.0)) return split_breakdown(B, it, sh);
   phase_split_update<D>(B, lb, blockIdx.x, rho / pq, beta, v, sh);
   if (lead) st->itv[parity ^ 1] = it + 1;
 }
@@ -372,8 +376,10 @@ __global__ __launch_bounds__(kNT) void k_split_check(PcgBuffers B, int parity) {
   __shared__ double sh[kNT / 64];
   const double rr = reduce_partials(B.part2 + B.nblocks, B.nblocks, sh);
   if (threadIdx.x == 0) {
-    B.st->it = B.st->itv[parity];
-    (void)split_goes_on(B, B.st->it, rr, true);
+    PcgState* st = B.st;
+    st->rr = rr;
+    st->it = st->itv[parity];
+    (void)split_goes_on(B, st->it, rr, true);
   }
 }
 
@@ -869,7 +875,7 @@ __global__ __launch_bounds__(kNT) void k_split_persistent(PcgBuffers B, GridBarr
     if (!grid_barrier(bar, &s_flag)) break;
     const double pq = reduce_partials(B.part1, nlb, sh);
     if (!(pq > 0.0)) {
-      split_breakdown(B, it, lead);
+      split_breakdown(B, it, sh);
       break;
     }
     // the update's logical workgroups likewise
