@@ -320,26 +320,29 @@ int cached_variant(const gf_ell* m) {
 }
 
 namespace {
-// ms of a whole iteration with variant v (unpreconditioned, from a scattered
-// right-hand side); negative where that system breaks down
-int time_iteration(gf_ctx* ctx, gf_ell* m, int v, int reps, double* ms) {
+// ms of a whole iteration with variant v, the best of three runs (unpreconditioned,
+// from a scattered right-hand side); negative where that system breaks down
+int time_iteration(gf_ctx* ctx, gf_ell* m, int v, double* ms) {
   const int st = prepare_variant(ctx, m, v);
   if (st) return st;
   set_variant(m, v);
-  PcgBuffers B = make_buffers(m, nullptr);
-  B.single = false;  // faster than two launches where it fits: it need not be timed
+  const PcgBuffers B = make_buffers(m, nullptr);
   GF_HIP_CHECK(ctx, launch_probe_setup(ctx->stream, B, m->plan->wb));
-  for (int it = 0; it < 2; ++it)
-    GF_HIP_CHECK(ctx, launch_pcg_iteration(ctx->stream, B, it & 1));
-  GF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_start, ctx->stream));
-  for (int it = 0; it < reps; ++it)
-    GF_HIP_CHECK(ctx, launch_pcg_iteration(ctx->stream, B, it & 1));
-  GF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_stop, ctx->stream));
+  constexpr int kRun = 8;
+  double best = 1e300;
+  for (int run = -1; run < 3; ++run) {  // the first one warms up
+    GF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_start, ctx->stream));
+    for (int it = 0; it < kRun; ++it)
+      GF_HIP_CHECK(ctx, launch_pcg_iteration(ctx->stream, B, it & 1));
+    GF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_stop, ctx->stream));
+    GF_HIP_CHECK(ctx, hipEventSynchronize(ctx->ev_stop));
+    float t = 0.f;
+    GF_HIP_CHECK(ctx, hipEventElapsedTime(&t, ctx->ev_start, ctx->ev_stop));
+    if (run >= 0) best = std::min(best, double(t) / kRun);
+  }
   PcgHostState h;
   GF_HIP_CHECK(ctx, read_pcg_state(ctx->stream, B, &h));
-  float t = 0.f;
-  GF_HIP_CHECK(ctx, hipEventElapsedTime(&t, ctx->ev_start, ctx->ev_stop));
-  *ms = h.done ? -1.0 : double(t) / reps;
+  *ms = h.done ? -1.0 : best;
   return GF_OK;
 }
 }  // namespace
@@ -363,6 +366,7 @@ int tune_spmv(gf_ctx* ctx, gf_ell* m, int force, double* ms_out, int* chosen) {
   // compare by it
   double best[2] = {1e300, 1e300};  // three launches an iteration, two launches
   int best_v[2] = {kThreadU8, -1};
+  bool single = false;  // the two launches are one of one workgroup
   for (int v = 0; v < kNumSpmvVariants; ++v) {
     if (!variant_fits(m, v)) {
       if (ms_out) ms_out[v] = -1.0;
@@ -385,13 +389,16 @@ int tune_spmv(gf_ctx* ctx, gf_ell* m, int force, double* ms_out, int* chosen) {
       best[two] = avg;
       best_v[two] = v;
     }
+    single |= B.single;
   }
   int pick = best_v[0];
-  if (best_v[1] >= 0) {
+  if (single) {
+    pick = best_v[1];  // by single_fits' measurements: fractions of any launch
+  } else if (best_v[1] >= 0) {
     // whole iterations: the two launches form the direction in both of theirs
     double ms[2];
     for (int k = 0; k < 2; ++k)
-      if ((st = time_iteration(ctx, m, best_v[k], reps, &ms[k]))) return st;
+      if ((st = time_iteration(ctx, m, best_v[k], &ms[k]))) return st;
     const double* t = ms[0] >= 0.0 && ms[1] >= 0.0 ? ms : best;
     pick = best_v[t[1] <= t[0] ? 1 : 0];
   }
@@ -401,10 +408,10 @@ int tune_spmv(gf_ctx* ctx, gf_ell* m, int force, double* ms_out, int* chosen) {
 }
 
 // The variant of a solve whose caller chose none: the slice-group variant
-// untimed for a matrix that stays in the last-level cache, whose two-launch
-// iteration is the fastest on every size measured (Q4 64x32 to Brick20 24^3;
-// timing eleven variants took 12 ms of an 89 ms analysis of Q8 201x67), else
-// the fastest by measurement.
+// untimed for a matrix that stays in the last-level cache (iter_variant), whose
+// two-launch iteration is the fastest on every size measured there (timing eleven
+// variants took 12 ms of an 89 ms analysis of Q8 201x67), else the fastest by
+// measurement.
 int choose_variant(gf_ctx* ctx, gf_ell* m) {
   int st = ensure_plan(ctx, m);
   if (st || m->plan->variant >= 0) return st;

@@ -222,6 +222,14 @@ for update, want in ((20.0, False), (2.0, True)):
     assert (chosen == 9) == want, (chosen, ms)
     # 16 products and one launch that readies the state
     assert abs(ms[0] - 6.0e-3) < 1e-4 and abs(ms[9] - 5.0e-3) < 1e-4, ms
+
+# a system for one workgroup takes it whatever its two launches would cost
+p = P.structured(gf.GF_Q4, 20, 10)
+fake.fake_cost(b"k_split_product", 50.0)
+mesh = mesh_of(p)
+K = ctx.symbolic(mesh)
+ctx.assemble(mesh, K)
+assert ctx.tune(K)[0] == 9
 """)
 
 
