@@ -260,6 +260,8 @@ hipError_t launch_pcg_iteration_timed(hipStream_t s, const PcgBuffers& B, int pa
 // iterations between two looks at the state from the host (even), and of a
 // launch of the single workgroup
 constexpr int kPcgChunk = 32, kSingleChunk = 512;
+// count iterations (even; kSingleChunk at most), from one of parity 0 on
+hipError_t launch_pcg_run(hipStream_t s, const PcgBuffers& B, int count);
 // such a chunk, and the state it left
 hipError_t launch_pcg_chunk(hipStream_t s, const PcgBuffers& B);
 // after iterations, the next of which has this parity: the state they left

@@ -332,8 +332,7 @@ int time_iteration(gf_ctx* ctx, gf_ell* m, int v, double* ms) {
   double best = 1e300;
   for (int run = -1; run < 3; ++run) {  // the first one warms up
     GF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_start, ctx->stream));
-    for (int it = 0; it < kRun; ++it)
-      GF_HIP_CHECK(ctx, launch_pcg_iteration(ctx->stream, B, it & 1));
+    GF_HIP_CHECK(ctx, launch_pcg_run(ctx->stream, B, kRun));
     GF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_stop, ctx->stream));
     GF_HIP_CHECK(ctx, hipEventSynchronize(ctx->ev_stop));
     float t = 0.f;
@@ -362,19 +361,20 @@ int tune_spmv(gf_ctx* ctx, gf_ell* m, int force, double* ms_out, int* chosen) {
   }
   GF_HIP_CHECK(ctx, hipMemsetAsync(P->p, 0, size_t(m->n) * sizeof(double), ctx->stream));
   const int reps = m->n > 200000 ? 10 : 16;
-  // the product of every variant; those whose iterations differ in nothing else
-  // compare by it
-  double best[2] = {1e300, 1e300};  // three launches an iteration, two launches
-  int best_v[2] = {kThreadU8, -1};
-  bool single = false;  // the two launches are one of one workgroup
+  // the product of every variant with three launches an iteration, which differ in
+  // nothing else
+  double best = 1e300;
+  int best_v = kThreadU8, two = -1;
   for (int v = 0; v < kNumSpmvVariants; ++v) {
-    if (!variant_fits(m, v)) {
-      if (ms_out) ms_out[v] = -1.0;
-      continue;
-    }
+    if (ms_out) ms_out[v] = -1.0;
+    if (!variant_fits(m, v)) continue;
     if ((st = prepare_variant(ctx, m, v))) return st;
     set_variant(m, v);
     PcgBuffers B = make_buffers(m, nullptr);
+    if (is_split_variant(B.iter_variant)) {
+      two = v;
+      continue;
+    }
     GF_HIP_CHECK(ctx, launch_spmv_pq_repeat(ctx->stream, B, 2));
     GF_HIP_CHECK(ctx, hipEventRecord(ctx->ev_start, ctx->stream));
     GF_HIP_CHECK(ctx, launch_spmv_pq_repeat(ctx->stream, B, reps));
@@ -384,26 +384,23 @@ int tune_spmv(gf_ctx* ctx, gf_ell* m, int force, double* ms_out, int* chosen) {
     GF_HIP_CHECK(ctx, hipEventElapsedTime(&ms, ctx->ev_start, ctx->ev_stop));
     const double avg = double(ms) / reps;
     if (ms_out) ms_out[v] = avg;
-    const int two = is_split_variant(B.iter_variant) ? 1 : 0;
-    if (avg < best[two]) {
-      best[two] = avg;
-      best_v[two] = v;
+    if (avg < best) {
+      best = avg;
+      best_v = v;
     }
-    single |= B.single;
   }
-  int pick = best_v[0];
-  if (single) {
-    pick = best_v[1];  // by single_fits' measurements: fractions of any launch
-  } else if (best_v[1] >= 0) {
-    // whole iterations: the two launches form the direction in both of theirs
-    double ms[2];
-    for (int k = 0; k < 2; ++k)
-      if ((st = time_iteration(ctx, m, best_v[k], &ms[k]))) return st;
-    const double* t = ms[0] >= 0.0 && ms[1] >= 0.0 ? ms : best;
-    pick = best_v[t[1] <= t[0] ? 1 : 0];
+  if (two >= 0) {
+    // two launches (or one workgroup) divide the work otherwise: whole iterations are
+    // compared, and the difference is what its product is better or worse by
+    double it3 = -1.0, it2 = -1.0;
+    if ((st = time_iteration(ctx, m, best_v, &it3)) || (st = time_iteration(ctx, m, two, &it2)))
+      return st;
+    const double avg = it3 >= 0.0 && it2 >= 0.0 ? std::max(best + it2 - it3, 1e-4) : best;
+    if (ms_out) ms_out[two] = avg;
+    if (avg <= best) best_v = two;
   }
-  set_variant(m, pick);
-  if (chosen) *chosen = pick;
+  set_variant(m, best_v);
+  if (chosen) *chosen = best_v;
   return GF_OK;
 }
 

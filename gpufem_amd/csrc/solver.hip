@@ -1175,10 +1175,16 @@ hipError_t launch_pcg_iteration(hipStream_t s, const PcgBuffers& B, int parity) 
   return e != hipSuccess ? e : launch_updates(s, B, parity);
 }
 
-hipError_t launch_pcg_chunk(hipStream_t s, const PcgBuffers& B) {
-  if (B.single) return launch_single(s, B, kSingleChunk);
+hipError_t launch_pcg_run(hipStream_t s, const PcgBuffers& B, int count) {
+  if (B.single) return launch_single(s, B, count);
   hipError_t e = hipSuccess;
-  for (int it = 0; it < kPcgChunk && e == hipSuccess; ++it) e = launch_pcg_iteration(s, B, it & 1);
+  for (int it = 0; it < count && e == hipSuccess; ++it) e = launch_pcg_iteration(s, B, it & 1);
+  return e;
+}
+
+hipError_t launch_pcg_chunk(hipStream_t s, const PcgBuffers& B) {
+  if (B.single) return launch_pcg_run(s, B, kSingleChunk);
+  const hipError_t e = launch_pcg_run(s, B, kPcgChunk);
   return e != hipSuccess ? e : launch_pcg_check(s, B, 0);
 }
 

@@ -318,14 +318,15 @@ int gf_pcg(gf_ctx* ctx, gf_ell* m, const double* b, double* x, int32_t nrhs,
  * slices of unequal length).  Variants 0..2 and 5..10 add each row's entries
  * in slot order and give bitwise-identical products.  force_variant >= 0 fixes a
  * variant; -1 times the product of every variant that fits this matrix and
- * keeps the fastest (9/10 on a matrix that stays in the last-level cache: against
- * the fastest of the others by whole iterations).  gf_pcg does this on first use, but takes 9/10 untimed for a
+ * keeps the fastest.  gf_pcg does this on first use, but takes 9/10 untimed for a
  * mesh matrix that stays in the last-level cache: there its iteration is two
  * launches, several waves share a slice, and the sums agree with the variant's
  * products to rounding (a small system: one launch of one workgroup for many
  * iterations, whatever the schedule).  ms_per_variant (may be NULL)
- * receives GF_SPMV_VARIANTS average times of the product (-1 for variants that do not fit).  No
- * reference counterpart; it plays the role of SetOclStrategy /
+ * receives GF_SPMV_VARIANTS average times of the product (-1 for variants that do
+ * not fit; for 9/10 on a matrix that stays in the last-level cache the fastest
+ * other's product plus what its whole iteration differs by from that one's, at
+ * least 1e-4).  No reference counterpart; it plays the role of SetOclStrategy /
  * SetOclLocalSize (src/SPRmatrix/SPRmatrix.h:110-121) chosen by measurement
  * instead of by hand. */
 #define GF_SPMV_VARIANTS 11
