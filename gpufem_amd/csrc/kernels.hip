@@ -1119,10 +1119,13 @@ hipError_t launch_gather_cfg(hipStream_t s, const GArgs& g) {
 //      incidence) at two waves per SIMD, Gauss-point loop rolled: 101x90x88
 //      1.36 ms, over the stored geometry 1.56; neighbours in chunks of 4 with
 //      two points unrolled 1.42 and 1.87, two points unrolled and 8 neighbours
-//      1.8, three waves 1.6 or more.  Then 54 % of the cycles issue vector
-//      instructions (FP64 mostly) and 36 % wait for loads.  Row units (one row
-//      per unit, each element's geometry once per row) took 1.6 times the node
-//      units with 2 lanes per row, 2.4 with one lane per row.
+//      1.8, three waves 1.6 or more.  Then vector instructions (FP64 mostly, 24
+//      TFLOP/s) take 43 % of the issue time and a wave waits 55 % of its own.
+//      With 27 Gauss points (chunks of 4, two points unrolled, the same two
+//      waves per SIMD) 60^3 takes 0.88 ms, 0.92 with the registers left to the
+//      compiler and the lanes in turns, over the stored geometry 1.17 and 1.20.
+//      Row units (one row per unit, each element's geometry once per row) took
+//      1.6 times the node units with 2 lanes per row, 2.4 with one lane per row.
 //  Brick20: row units, 4 lanes per row (256 VGPRs + AGPRs): 48^3 8.1-8.7 ms;
 //      node units need chunks of at most 4 neighbours for their registers and
 //      recompute the 20-node geometry per chunk (10.8-20.5 ms).

@@ -643,7 +643,13 @@ hipError_t launch_conv(hipStream_t s, const ConvArgs& a) {
       a.in_off + a.cin > a.in_ld || a.out_off + a.cout > a.out_ld)
     return hipErrorInvalidValue;
   // 64 voxels per wave reuse a weight fragment four times; from about two waves
-  // per SIMD of 256 CUs down, the four waves of a workgroup share the voxels
+  // per SIMD of 256 CUs down, the four waves of a workgroup share the voxels, and
+  // below that take fewer of them.  us, by `waves`, 64 voxels a wave / 64, 32 and 16
+  // shared by four: 4,357 (65x65x33, 64 -> 128 channels) 181 / 173 163 217; 2,178
+  // (96 -> 32) 89 / 104 90 121, (16 -> 16) 17 / 15 20 31; 1,106 (32 -> 32) 26 / 19 20
+  // 29; 561 (32 -> 32) 24 / 12.0 12.2 17; 289 24 / 10 8.7 11; 149 24 / 9.2 7.6 7.8;
+  // 76 24 / 8.3 7.5 6.6.  Within 20 % of the best of them on every pair of channel
+  // counts the network has.
   const int64_t total = int64_t(a.batch) * a.vout.nodes();
   const int nct = a.cout >> 4, ct = nct % 4 == 0 ? 4 : nct % 3 == 0 ? 3 : nct % 2 == 0 ? 2 : 1;
   const int64_t waves = total * (nct / ct) / 64;
@@ -669,7 +675,9 @@ int wgrad_co_tiles(int cout) {
 
 int wgrad_chunks(int64_t voxels, int cin, int cout) {
   // about two workgroups per CU of 256 with the channel blocks, and at least
-  // two tiles of voxels each
+  // two tiles of voxels each; half / this / twice as many, us with the sum of the
+  // parts: 65x33x33, 192 -> 64 channels 260 / 229 / 250, 32 -> 32 38 / 30 / 39; 33^3,
+  // 64 -> 128 96 / 88 / 111; up to 17^3 all alike
   const int64_t blocks = int64_t(cin >> 4) * ((cout >> 4) / wgrad_co_tiles(cout));
   const int64_t tiles = (voxels + kWgTile - 1) / kWgTile;
   int64_t c = 512 / blocks;
