@@ -634,14 +634,15 @@ static bool tensors_fit(const gf_mesh* mesh, double share) {
 // only from plenty: the solvers' workspaces are allocated after them.
 static int small_mesh_variant(gf_ctx* ctx, const gf_mesh* mesh, gf_ell* m) {
   if (mesh->dim != 3 || !gather_fits(mesh, m)) return 0;
-  int v = 0;
-  if (ensure_n2e(ctx, mesh, m) == hipSuccess) {
-    v = 3;
-    if (mesh->type == GF_BRICK20 && tensors_fit(mesh, 0.125) &&
-        ensure_tensors(mesh, m) == hipSuccess)
-      v = 2;
+  int v = 3;
+  hipError_t e = ensure_n2e(ctx, mesh, m);
+  if (e != hipSuccess) {
+    v = 0;
+  } else if (mesh->type == GF_BRICK20 && tensors_fit(mesh, 0.125)) {
+    e = ensure_tensors(mesh, m);
+    if (e == hipSuccess) v = 2;
   }
-  (void)hipGetLastError();  // a failed allocation is no error of the call
+  if (e != hipSuccess) (void)hipGetLastError();  // no error of this call
   return v;
 }
 
